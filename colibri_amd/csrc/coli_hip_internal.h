@@ -121,28 +121,30 @@ struct ColiGemvArgs {
 };
 
 
-// Grouped GEMM (prefill): problems of many rows, tiled 64 rows x
+// Grouped GEMM (prefill): problems of many rows, tiled COLI_GM_TILE rows x
 // COLI_GM_BLOCK_TILES row tiles (half as many gate/up pairs when dual) with
 // the activation fragments staged in LDS. COLI_GM_WAVES: the block-scaled
 // variant (gemm_mx.hip), 8 waves x 2 row tiles.
 #define COLI_GM_WAVES 8
 #define COLI_GM_BLOCK_TILES 16
 #ifndef COLI_GM_ROWS
-#define COLI_GM_ROWS 64
+#define COLI_GM_ROWS 64     // rows of a short tile (and of the block-scaled variant's tiles)
 #endif
+#define COLI_GM_TILE 128    // rows of a work item of coli_gemm_tiles
 
 struct ColiGemmArgs {
-    const ColiProb *prob;
+    const ColiProb *prob;     // device descriptors; null: the single problem prob0 (item i = its row tile i)
+    ColiProb prob0;
     const int *nprob_dev;     // live problems (device); null: nprob
     int nprob;
-    const int *mt_list;       // work list of (problem << 16 | row tile); null: tile i of problem 0..
+    const int *mt_list;       // work list of (problem << 16 | row tile)
     const int *n_mt_dev;      // live entries of mt_list (device)
     int n_mt;                 // upper bound of the list (grid sizing)
     int nrt, nq, O;
     int rb_per_prob;          // output blocks of COLI_GM_WAVES x 2 row tiles (dual: x 1 gate + 1 up)
     const int *xrows;         // fragment row of batch row r = xrows[xrow_off + r] (null: xrow_off + r)
     const _Float16 *xhi, *xlo;
-    int xstride;              // halves per fragment row
+    int xstride;              // halves per fragment row (= ngp * 32)
     const int *xexp;
     const int *haslo;
     int lo_gen;
@@ -151,6 +153,9 @@ struct ColiGemmArgs {
     int ldo;
     float swiglu_limit;       // > 0: DeepSeek-V4 clamped SwiGLU in the DUAL epilogue
     int fold;                 // MXFP4, every matrix e8_fold: scales folded into the unpacked operand
+    int splits, qps;          // K split: quads per split; 1: none
+    float *partial;           // [split][part_rows][rb_per_prob * 256] raw sums (splits > 1)
+    int part_rows;            // output rows of the call (splits > 1: fragment row r is output row r)
 };
 
 // Grouped MXFP4 GEMM on the block-scaled MFMA (gemm_mx.hip): activations as

@@ -383,16 +383,44 @@ int run_gemv(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     return hip_check(coli_launch_gemv(kind, &a, pl.R, dual ? 1 : 0, pl.W, max_rows, ctx->stream), "gemv launch");
 }
 
+// K splits of a grouped GEMM whose work list the host knows, and its time in
+// us: `items` row tiles of at most `tile` rows x rb blocks over nq quads,
+// `rows` output rows of `cols` partial sums each. One workgroup fills a CU, so
+// a launch takes whole rounds of one workgroup per CU; splitting K levels them
+// (and fills a chip that the blocks alone leave idle) for the partials' round
+// trip and the reduction launch. Measured: a workgroup takes about 10 us and
+// 2.5 us a quad on a tall tile, 1.3 us on a short one (224 workgroups of 128 x
+// 256: 11.4 / 20.7 / 95 us at 1 / 4 / 32 quads); the reduction launch about 5
+// us and the partials' bytes, written and read, at about 4 TB/s.
+static double gemm_plan(const DevCtx *ctx, long items, int rb, int nq, int tile, long rows, long cols, int *splits) {
+    const long cus = ctx && ctx->cu_count ? ctx->cu_count : 256;
+    const double tq = tile > COLI_GM_ROWS ? 2.5 : 1.3;
+    double best = 0.0;
+    for (int s = 1; s <= 16 && (s == 1 || nq / s >= 4); s++) {
+        const double us = (double)((items * rb * s + cus - 1) / cus) * (10.0 + (nq + s - 1) / s * tq) +
+                          (s > 1 ? 5.0 + (double)s * rows * cols * 8 / 4e6 : 0.0);
+        if (s == 1 || us < best) {
+            *splits = s;
+            best = us;
+        }
+    }
+    return best;
+}
+
 // Grouped GEMM over problems of many rows (see gemm.hip); mt_list_dev holds
-// n_mt entries (problem << 16 | 64-row tile), problem indices relative to
-// probs_dev.
+// n_mt entries (problem << 16 | row tile), problem indices relative to
+// probs_dev. inline_prob: the single problem instead of descriptors and list.
+// split_rows > 0: the launch covers output rows [0, split_rows) whole, in
+// fragment-row order, n_mt is exact and K may be split across workgroups.
 int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int nprob, const int *nprob_dev,
              const int *mt_list_dev, const int *n_mt_dev, int n_mt, int nrt, int nq, int O, int set,
-             const int *xrows_dev, float *out, int ldo, float swiglu_limit, bool fold) {
+             const int *xrows_dev, float *out, int ldo, float swiglu_limit, bool fold, const ColiProb *inline_prob,
+             int split_rows) {
     if (n_mt <= 0) return 1;
     FragSet &f = ctx->frag[set];
-    if (!(kind == COLI_KIND_FP4 && mx_gemm_enabled()) && !flush_frags(ctx, set)) return 0;
-    if (kind == COLI_KIND_FP4 && mx_gemm_enabled()) {
+    const bool mx = kind == COLI_KIND_FP4 && !inline_prob && mx_gemm_enabled();
+    if (!mx && !flush_frags(ctx, set)) return 0;
+    if (mx) {
         ColiGemmMxArgs m;
         std::memset(&m, 0, sizeof(m));
         m.prob = probs_dev;
@@ -420,6 +448,10 @@ int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     ColiGemmArgs a;
     std::memset(&a, 0, sizeof(a));
     a.prob = probs_dev;
+    if (inline_prob) {
+        a.prob = nullptr;
+        a.prob0 = *inline_prob;
+    }
     a.nprob_dev = nprob_dev;
     a.nprob = nprob;
     a.mt_list = mt_list_dev;
@@ -437,11 +469,27 @@ int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     a.xexp = (const int *)f.exp.p;
     a.haslo = (const int *)ctx->flags.p + set;
     a.lo_gen = f.gen;
+    if (f.nolo) {   // a zero word never reaches generation 1
+        a.haslo = (const int *)ctx->zeros.p;
+        a.lo_gen = 1;
+    }
     a.zero = (const uint8_t *)ctx->zeros.p;
     a.out = out;
     a.ldo = ldo;
     a.swiglu_limit = swiglu_limit;
     a.fold = fold && kind == COLI_KIND_FP4;
+    a.splits = 1;
+    if (split_rows > 0 && split_rows <= 65535) {
+        const long cols = (long)a.rb_per_prob * COLI_GM_BLOCK_TILES * 16;
+        gemm_plan(ctx, n_mt, a.rb_per_prob, nq, std::min(split_rows, COLI_GM_TILE), split_rows, cols, &a.splits);
+        a.part_rows = split_rows;
+        if (a.splits > 1) {
+            if (!reserve(ctx, &ctx->partial, (size_t)a.splits * split_rows * cols * sizeof(float), 0)) return 0;
+            a.partial = (float *)ctx->partial.p;
+        }
+    }
+    a.qps = (nq + a.splits - 1) / a.splits;
+    a.splits = (nq + a.qps - 1) / a.qps;
     return hip_check(coli_launch_gemm(kind, dual ? 1 : 0, &a, ctx->stream), "gemm launch");
 }
 
@@ -538,16 +586,17 @@ static int run_expert_group(DevCtx *ctx, const Member *m, int count, int total, 
     }
     (void)t0g; (void)t0d; (void)split_first;
     // Members of many rows go through the grouped GEMM: one work list of
-    // (problem, 64-row tile) per launch, uploaded after the descriptors.
+    // (problem, row tile) per launch, uploaded after the descriptors.
     const bool use_gemm = max_rows > COLI_GEMM_MIN_ROWS;
     std::vector<int> mt;
     std::vector<int> mt_first(launches.size(), 0), mt_count(launches.size(), 0);
     if (use_gemm)
         for (size_t l = 0; l < launches.size(); l++) {
             mt_first[l] = (int)mt.size();
+            const int tile = launches[l].kind == COLI_KIND_FP4 && mx_gemm ? COLI_GM_ROWS : COLI_GM_TILE;
             for (int q = 0; q < launches[l].n; q++) {
                 const int rows = probs[launches[l].first + q].nrows;
-                for (int t = 0; t * COLI_GM_ROWS < rows; t++) mt.push_back(q << 16 | t);
+                for (int t = 0; t * tile < rows; t++) mt.push_back(q << 16 | t);
             }
             mt_count[l] = (int)mt.size() - mt_first[l];
         }
@@ -570,7 +619,8 @@ static int run_expert_group(DevCtx *ctx, const Member *m, int count, int total, 
         const Launch &L = launches[l];
         if (use_gemm)
             return run_gemm(ctx, L.kind, dual, pdev + L.first, L.n, nullptr, mtdev + mt_first[l], nullptr,
-                            mt_count[l], L.nrt, L.nq, L.O, L.set, nullptr, L.out, L.ldo, 0.0f, fold);
+                            mt_count[l], L.nrt, L.nq, L.O, L.set, nullptr, L.out, L.ldo, 0.0f, fold, nullptr,
+                            L.n == count ? total : 0);
         return run_gemv(ctx, L.kind, dual, pdev + L.first, L.n, nullptr, L.nrt, L.nq, L.O, max_rows, L.set,
                         nullptr, L.out, L.ldo, nullptr, 0.0f, nullptr, nullptr, fold);
     };
@@ -803,6 +853,32 @@ void forget_emitted(DevCtx *ctx, const void *dst, size_t bytes) {
     }
 }
 
+// The same product for more rows than one batch tile of the GEMV: the
+// grouped GEMM on one problem (14336 x 4096 int4 with its fragment build: 33
+// rows 36 -> 27 us, 512 rows 301 -> 123 us).
+static int gemm_rows(DevCtx *ctx, ColiCudaTensor *t, const void *sc, int set, float *y_dev, int S, bool fold) {
+    const ColiProb p = {t->w, sc, nullptr, nullptr, S, 0, 0, 0};
+    return run_gemm(ctx, t->kind, false, nullptr, 1, nullptr, nullptr, nullptr, (S + COLI_GM_TILE - 1) / COLI_GM_TILE,
+                    t->nrt, t->nq, t->O, set, nullptr, y_dev, t->O, 0.0f, fold, &p, S);
+}
+
+// Whether S rows of t run the GEMM: beyond one 16-row batch tile, when its
+// modelled time is below the GEMV's, which streams the matrix again for every
+// batch tile at about 3 TB/s (0.36 us a tile and MB, measured from 512 x 2048
+// to 14336 x 4096). Crossovers measured (GEMV / GEMM): 4096 x 14336 17 rows 41
+// / 31 us; 14336 x 4096 32 rows 29 / 27; 4096 x 4096 128 rows 30 / 35, 192
+// rows 42 / 40; 2048 x 7168 128 rows 28 / 37, 192 rows 46 / 40; 512 x 2048
+// 1024 rows 28 / 39.
+static bool dense_on_gemm(const DevCtx *ctx, const ColiCudaTensor *t, int S) {
+    if (S <= 16 || S > 65535) return S > 16;
+    const int rb = (t->nrt + COLI_GM_BLOCK_TILES - 1) / COLI_GM_BLOCK_TILES;
+    int splits;
+    const double gemm = gemm_plan(ctx, (S + COLI_GM_TILE - 1) / COLI_GM_TILE, rb, t->nq, std::min(S, COLI_GM_TILE), S,
+                                  (long)rb * COLI_GM_BLOCK_TILES * 16, &splits);
+    const double gemv = 5.0 + 0.36 * ((S + 15) / 16) * (double)(t->w_bytes + t->sc_bytes) / 1e6;
+    return gemm < gemv;
+}
+
 // GEMV of t over the prepared fragments of S rows -> y_dev[S, O]; the
 // problem travels in the kernel arguments (no descriptor, no host sync).
 // With next: y_dev is also emitted as next's input fragments (set 2 / 3).
@@ -811,6 +887,7 @@ static int gemm_run(DevCtx *ctx, ColiCudaTensor *t, float *y_dev, int S, const C
     const int set = ctx->dense_set[t->kind == COLI_KIND_FP4 ? 1 : 0];
     const bool fold = t->kind == COLI_KIND_FP4 && t->e8_fold;
     forget_emitted(ctx, y_dev, (size_t)S * t->O * sizeof(float));
+    if (dense_on_gemm(ctx, t, S)) return gemm_rows(ctx, t, t->sc, set, y_dev, S, fold);
     if (!next) {
         return run_gemv(ctx, t->kind, false, nullptr, 1, nullptr, t->nrt, t->nq, t->O, S, set, nullptr, y_dev, t->O,
                         &p, 0.0f, nullptr, nullptr, fold);
@@ -920,8 +997,9 @@ static int idot_dev(DevCtx *ctx, ColiCudaTensor *t, float *y_dev, const float *x
                    "int8 activation rows"))
         return 0;
     const ColiProb p = {t->w, t->sc_unit, nullptr, nullptr, S, 0, 0, 0};
-    if (!run_gemv(ctx, t->kind, false, nullptr, 1, nullptr, t->nrt, t->nq, t->O, S, set, nullptr,
-                  (float *)ctx->idot_y.p, t->O, &p))
+    if (dense_on_gemm(ctx, t, S) ? !gemm_rows(ctx, t, t->sc_unit, set, (float *)ctx->idot_y.p, S, false)
+                               : !run_gemv(ctx, t->kind, false, nullptr, 1, nullptr, t->nrt, t->nq, t->O, S, set,
+                                           nullptr, (float *)ctx->idot_y.p, t->O, &p))
         return 0;
     forget_emitted(ctx, y_dev, (size_t)S * t->O * sizeof(float));
     return hip_check(coli_launch_idot_scale(y_dev, (const float *)ctx->idot_y.p, (const float *)ctx->idot_sx.p, t->sc,

@@ -1,13 +1,18 @@
 // gemm.hip -- grouped dequant-fused GEMM for gfx950: many-row problems
-// (prefill chunks, verification batches), y[b, o] = sum_g scale[o, g] *
-// sum_{k in g} x[b, k] w[o, k], the same arithmetic as the GEMV (c/quant.h
-// fmt=4 and fmt=7) with the weights read once per 64 rows instead of once per
-// 16.
+// (prefill chunks, verification batches, dense matrices of many rows), y[b, o]
+// = sum_g scale[o, g] * sum_{k in g} x[b, k] w[o, k], the same arithmetic as
+// the GEMV (c/quant.h fmt=4 and fmt=7) with the weights read once per 128 rows
+// instead of once per 16.
 //
-// Work item = (problem, 64-row tile, output block of COLI_GM_BLOCK_TILES row
-// tiles). A workgroup of COLI_GM_W waves gives each wave R = COLI_GM_BLOCK_TILES
-// / COLI_GM_W weight tiles (DUAL: gate/up pairs of the same 16 output rows,
-// SwiGLU in the epilogue) over the full K, one 128-column quad per step:
+// Work item = (problem, 128-row tile, output block of COLI_GM_BLOCK_TILES row
+// tiles, K split). Tiles of more than 64 rows run gemm_tall below (their
+// bound is the matrix cores and the issue slots); shorter ones, whose bound is
+// the weight stream, the loop described here. A K split (only where the host
+// knows the work list: gemm_plan, expert.hip) leaves raw partial sums that
+// coli_gemm_reduce adds in split order. A workgroup of COLI_GM_W waves gives
+// each wave R = COLI_GM_BLOCK_TILES / COLI_GM_W weight tiles (DUAL: gate/up
+// pairs of the same 16 output rows, SwiGLU in the epilogue) over its K, one
+// 128-column quad per step:
 //  * every load of the main loop is an LDS DMA into a ring of PD stages: each
 //    wave's weight tiles and their scales (private to the wave), and the
 //    quad's activation fragments of the tile's rows (fp16 hi + lo of x * 2^-E,
@@ -78,6 +83,267 @@ struct GmGeom {
 static_assert(GmGeom<COLI_KIND_I4_F>::pd(COLI_GM_ROWS / 16, true, GmGeom<COLI_KIND_I4_F>::kR / 2) >= 3,
               "the ring needs three stages");
 
+// Ring geometry of a tall tile (65-128 rows). Activations are staged per half
+// quad (2 groups x 8 subtiles), weights and scales per quad; the weights of
+// quad q are fetched with the activations of quad q - 1.
+template <int KIND>
+struct GtGeom {
+    static constexpr int kSub = COLI_GM_TILE / 16;
+    static constexpr int kHalf = 2 * kSub * 1024;                                       // one half quad, hi or lo
+    static constexpr int act(bool lo) { return kHalf * (lo ? 2 : 1); }
+    static constexpr int kWSlot = COLI_GM_BLOCK_TILES * (COLI_TILE_BYTES + ScaleGeom<KIND>::kBytes);
+    static constexpr int pd(bool lo) { return lo ? 3 : 5; }                             // activation stages
+    static constexpr int nw(bool lo) { return lo ? 2 : 3; }                             // weight slots
+    static constexpr int kScInst = COLI_GM_BLOCK_TILES * ScaleGeom<KIND>::kBytes / 1024;  // 1 KiB scale DMAs a quad
+    static constexpr int kExp = GmGeom<KIND>::kLds - 4096;   // the rows' exponents, 8 copies each
+    static_assert(act(true) * pd(true) + nw(true) * kWSlot <= kExp && act(false) * pd(false) + nw(false) * kWSlot <= kExp,
+                  "the rings must fit the LDS");
+};
+
+// Byte offset in a subtile's 2 KiB half quad of the 16 B that lane l of a
+// 32x32x16 operand reads for (group g, K half t): row l % 16, k-slice 2 t +
+// l / 32. A row's eight 16 B pieces are stored XORed with a key of the row, so
+// the sixteen lanes of a phase read sixteen different slots of 256 B.
+__device__ __forceinline__ int tall_key(int r) { return (r & 7) ^ (r >> 3); }
+__device__ __forceinline__ int tall_off(int lane, int g, int t) {
+    const int r = lane & 15;
+    return ((lane >> 4) & 1) * 2048 + r * 128 + 16 * ((4 * g + 2 * t + (lane >> 5)) ^ tall_key(r));
+}
+
+// One tall tile's pass over quads [0, nq): the workgroup's 8 waves are 2 (row
+// halves) x 4 (four weight tiles each); a wave computes NB 32-row blocks x two
+// 32-column blocks (tiles 2n, 2n + 1) on v_mfma_f32_32x32x16_f16, so every
+// activation it reads from LDS feeds four tiles (the short tiles' 1 x 8
+// arrangement: two) and an MFMA takes two issue slots for 32 cycles (the
+// 16x16x32 form: two for 16; the int4 loop is bound by its VALU and MFMA issue
+// slots). wt0, wt1: quad 0 of tiles wave, wave + 8 of the block; sp: this
+// lane's 16 B of the wave's scale DMA; xo0, xo1: this lane's 16 B of rows 16
+// wave + l / 8 and + 8 (one DMA covers 8 rows x 128 B: whole cache lines; 16
+// rows x 64 B ran at half the rate). store(row, tile of the block, gate or
+// plain value, value of the tile after it) takes the results.
+//
+// The loop is a sequence of steps, one per (group, row block, column block):
+// the step's 2 (4 with lo parts) MFMAs beside the work that needs no result of
+// theirs: the LDS reads of the next fragments, the scaling of the previous
+// step's products and a quarter of the next group's unpack. Left to itself the
+// compiler reads each fragment right before its use and waits for it.
+// (sched_barrier: nothing crosses a step; sched_group_barrier: MFMAs and VALU
+// work interleave inside it.) The ring is synchronized in the last step of
+// each half quad, whose own operands are in registers by then.
+// Measured (512 x 14336 x 4096 with lo parts, two MFMAs a product): int4 329 us
+// on the GEMV kernel, 155 us with the same tiles scheduled by the compiler,
+// 119-139 us here (1.0 PFLOP/s of MFMA work; 1.2 MXFP4; a bf16 library product
+// of 8192^3 reaches 1.4 on the card).
+template <int KIND, bool LO, bool FOLD, int NB, typename Store>
+__device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, const uint8_t *wt1, const uint8_t *sp,
+                                          const _Float16 *xhi, const _Float16 *xlo, uint32_t xo0, uint32_t xo1, int nq,
+                                          int lane, int wave, Store store) {
+    using T = GtGeom<KIND>;
+    using SG = ScaleGeom<KIND>;
+    constexpr int PD = T::pd(LO), NW = T::nw(LO), ACT = T::act(LO), WS = T::kWSlot;
+    constexpr int LA = LO ? 4 : 2;   // activation DMAs of a half quad and wave
+    uint8_t *const aring = lds, *const wring = lds + PD * ACT;
+    const int wm = wave >> 2, wn = wave & 3;
+    const int nh = 2 * nq;
+    // weights of quad q into weight slot ws, part (half): tile wave + 8 part,
+    // and with part 0 the scales
+    auto issue_w = [&](int q, uint8_t *ws, int part) {
+        q = min(q, nq - 1);
+        __builtin_amdgcn_global_load_lds((const void *)((part ? wt1 : wt0) + (size_t)q * COLI_TILE_BYTES + lane * 16),
+                                         (lds_void *)(ws + (wave + 8 * part) * COLI_TILE_BYTES), 16, 0, 0);
+        if (part == 0)
+            __builtin_amdgcn_global_load_lds((const void *)(sp + (size_t)q * SG::kBytes),
+                                             (lds_void *)(ws + COLI_GM_BLOCK_TILES * COLI_TILE_BYTES +
+                                                          (wave % T::kScInst) * 1024),
+                                             16, 0, 0);
+    };
+    // half quad h (part h & 1) into activation slot xs, and its share of the
+    // weights of quad h / 2 + 1 into slot ws. Past the end the last half quad
+    // is fetched again and nothing reads it: without a branch the loop's body
+    // is one basic block (across a branch the compiler sinks the scaling of
+    // the products to the end of the loop and spills them), and the counts of
+    // loads in flight stay fixed.
+    auto issue = [&](int h, uint8_t *xs, uint8_t *ws, int part) {
+        xs += wave * 2048;
+        const size_t o = (size_t)min(h, nh - 1) * 64;
+        __builtin_amdgcn_global_load_lds((const void *)(xhi + xo0 + o), (lds_void *)xs, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void *)(xhi + xo1 + o), (lds_void *)(xs + 1024), 16, 0, 0);
+        if constexpr (LO) {
+            __builtin_amdgcn_global_load_lds((const void *)(xlo + xo0 + o), (lds_void *)(xs + T::kHalf), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const void *)(xlo + xo1 + o), (lds_void *)(xs + T::kHalf + 1024), 16, 0, 0);
+        }
+        issue_w((h >> 1) + 1, ws, part);
+    };
+    // operands, all indices constant: the quad's tiles w[n][t] (the two K
+    // halves), reloaded for the next quad once unpacked; bw of this group and
+    // the next; fragments of this row block and the next; products of this
+    // step and the previous one
+    u32x4 w[2][2];
+    ScaleRegs<KIND> sc[2];
+    half8v bw[2][2][2], xh[2][2], xl[2][2];
+    float scl[2][2];
+    floatx16 d[2], acc[NB][2];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        d[1][i] = 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[b][0][i] = acc[b][1][i] = 0.0f;
+    }
+    const int l16 = (lane >> 4) & 1, wofs = l16 * COLI_TILE_BYTES + ((lane >> 5) * 16 + (lane & 15)) * 16;
+    auto load_w = [&](int n, int t, const uint8_t *ws) {
+        w[n][t] = *(const u32x4 *)(ws + (wn * 4 + 2 * n) * COLI_TILE_BYTES + t * 512 + wofs);
+    };
+    auto load_sc = [&](int n, const uint8_t *ws) {
+        sc[n].v = *(const decltype(sc[n].v) *)(ws + COLI_GM_BLOCK_TILES * COLI_TILE_BYTES +
+                                               (wn * 4 + 2 * n + l16) * SG::kBytes + (lane & 15) * sizeof(sc[n].v));
+    };
+    auto unpack = [&](int n, int t, int j) {
+        if (t == 0) scl[j & 1][n] = sc[n].get(j);
+        if constexpr (FOLD) bw[j & 1][n][t] = unpack_fp4_scaled(w[n][t][j], scl[j & 1][n]);
+        else bw[j & 1][n][t] = unpack_b<KIND>(w[n][t][j]);
+    };
+    const int xofs[2][2] = {{tall_off(lane, 0, 0), tall_off(lane, 0, 1)}, {tall_off(lane, 1, 0), tall_off(lane, 1, 1)}};
+    auto load_x = [&](int p, const uint8_t *xs, int g, int b) {   // group g (0, 1) of the half quad, row block b
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const uint8_t *q = xs + (2 * wm + b) * 4096 + xofs[g][t];
+            xh[p][t] = *(const half8v *)q;
+            if constexpr (LO) xl[p][t] = *(const half8v *)(q + T::kHalf);
+        }
+    };
+    auto scale = [&](auto pt, auto bt, auto nt, auto jt) {   // products d[p] of blocks (b, n), group parity jp
+        constexpr int p = decltype(pt)::value, b = decltype(bt)::value, n = decltype(nt)::value;
+        constexpr int jp = decltype(jt)::value;
+        if constexpr (!FOLD) {
+            floatx16 v = acc[b][n];
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = fmaf(d[p][i], scl[jp][n], v[i]);
+            acc[b][n] = v;
+        }
+    };
+    auto wait_lds = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+    auto barrier = [&]() {
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto aslot = [&](int k) { return aring + k * ACT; };
+    auto wslot = [&](int k) { return wring + k * WS; };
+    issue_w(0, wslot(0), 0);
+    issue_w(0, wslot(0), 1);
+#pragma unroll
+    for (int i = 0; i < PD - 1; i++)
+        issue(i, aslot(i), wslot(((i >> 1) + 1) % NW), i & 1);
+    constexpr int P0 = PD == 3 ? LA + 1 : 3 * LA + 4;   // stages 1 .. PD - 2
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P0) : "memory");
+    barrier();
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+        load_sc(n, wslot(0));
+        load_w(n, 0, wslot(0));
+        load_w(n, 1, wslot(0));
+    }
+    wait_lds();
+    barrier();   // weight slot 0 is free
+    issue(PD - 1, aslot(PD - 1), wslot((((PD - 1) >> 1) + 1) % NW), (PD - 1) & 1);
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+        unpack(n, 0, 0);
+        unpack(n, 1, 0);
+        scl[1][n] = 0.0f;
+    }
+    load_x(0, aslot(0), 0, 0);
+    int as = 0, wn1 = 1 % NW;        // activation slot of the half quad; weight slot of the next quad
+    int wi = ((PD >> 1) + 1) % NW;   // weight slot of the next issue (half quad PD)
+    // step (group j, row block b, column block n) of quad c; the tags keep
+    // every index constant
+    auto step = [&](int c, auto jt, auto bt, auto nt) {
+        constexpr int j = decltype(jt)::value, b = decltype(bt)::value, n = decltype(nt)::value;
+        constexpr int s = b * 2 + n, NS = 2 * NB;                    // step of the group
+        constexpr int p = (j * NB + b) & 1, dp = n;                  // parity of the fragments, of the products
+        constexpr int part = j >> 1;
+        constexpr bool lastb = b == NB - 1, half_end = lastb && (j & 1);
+        if constexpr (half_end && n == 1) {
+            // end of half quad h: its operands are read (their slot is free
+            // after the barrier), half quad h + 1 is waited for (stages h + 2
+            // .. h + PD - 1 stay in flight)
+            const int h = 2 * c + part;
+            constexpr int NP = PD == 3 ? (part ? LA + 1 : LA + 2) : 3 * LA + (part ? 4 : 5);
+            wait_lds();
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NP) : "memory");
+            barrier();
+            issue(h + PD, aslot(as), wslot(wi), (part + PD) & 1);
+            if ((part + PD) & 1) wi = wi == NW - 1 ? 0 : wi + 1;
+            as = as == PD - 1 ? 0 : as + 1;
+        }
+        // fragments of the next row block: in this block's first step, or
+        // after the ring's synchronization
+        if constexpr (half_end ? n == 1 : n == 0) load_x(p ^ 1, aslot(as), (lastb ? j + 1 : j) & 1, lastb ? 0 : b + 1);
+        floatx16 z = {};
+        if constexpr (FOLD) z = acc[b][n];
+#pragma unroll
+        for (int t = 0; t < 2; t++) z = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[p][t], bw[j & 1][n][t], z, 0, 0, 0);
+        if constexpr (LO) {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                z = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[p][t], bw[j & 1][n][t], z, 0, 0, 0);
+        }
+        if constexpr (FOLD) acc[b][n] = z;
+        else d[dp] = z;
+        // scale the previous step's products (n - 1 of this row block, or n =
+        // 1 of the one before)
+        constexpr int pb = n == 1 ? b : (b == 0 ? NB - 1 : b - 1), pj = n == 1 || b > 0 ? j : j + 3;
+        scale(std::integral_constant<int, dp ^ 1>{}, std::integral_constant<int, pb>{},
+              std::integral_constant<int, n ^ 1>{}, std::integral_constant<int, pj & 1>{});
+        // the next group's operands, 4 / NS of the four (n, t) a step, and of
+        // the next quad's tiles once the last group's are unpacked
+#pragma unroll
+        for (int k = s * (4 / NS); k < (s + 1) * (4 / NS); k++) {
+            unpack(k >> 1, k & 1, (j + 1) & 3);
+            if constexpr (j == 2) {
+                load_w(k >> 1, k & 1, wslot(wn1));
+                if (k & 1) load_sc(k >> 1, wslot(wn1));
+            }
+        }
+        // an MFMA first: the wait for this step's operands then comes before
+        // the next fragments' reads are queued behind them
+        constexpr int NM = LO ? 4 : 2, NV = FOLD ? 6 / NM : (16 + 12 * (4 / NS) + NM - 1) / NM;
+#pragma unroll
+        for (int k = 0; k < NM; k++) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, NV, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto group = [&](int c, auto jt) {
+        using C0 = std::integral_constant<int, 0>;
+        using C1 = std::integral_constant<int, 1>;
+        step(c, jt, C0{}, C0{});
+        step(c, jt, C0{}, C1{});
+        if constexpr (NB == 2) {
+            step(c, jt, C1{}, C0{});
+            step(c, jt, C1{}, C1{});
+        }
+    };
+    for (int c = 0; c < nq; c++) {
+        group(c, std::integral_constant<int, 0>{});
+        group(c, std::integral_constant<int, 1>{});
+        group(c, std::integral_constant<int, 2>{});
+        group(c, std::integral_constant<int, 3>{});
+        wn1 = wn1 == NW - 1 ? 0 : wn1 + 1;
+    }
+    scale(std::integral_constant<int, 1>{}, std::integral_constant<int, NB - 1>{}, std::integral_constant<int, 1>{},
+          std::integral_constant<int, 1>{});
+    // the last DMAs write this workgroup's LDS: none may outlive it
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // lane l, register i: row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            store(wm * 64 + b * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3), 4 * wn + l16, acc[b][0][i], acc[b][1][i]);
+}
+
 template <int KIND, bool DUAL>
 __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a) {
     using G = GmGeom<KIND>;
@@ -91,16 +357,116 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
     // (tile indices, validity, base pointers) stays in scalar registers.
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-    const int item = blockIdx.x / a.rb_per_prob, rb = blockIdx.x - item * a.rb_per_prob;
+    const int part = blockIdx.x / a.rb_per_prob, rb = blockIdx.x - part * a.rb_per_prob;
+    const int item = part / a.splits, split = part - item * a.splits;
     if (a.n_mt_dev && item >= *a.n_mt_dev) return;
     if (item >= a.n_mt) return;
-    const int tag = a.mt_list[item];
-    const int p = tag >> 16, mt = tag & 0xffff;
-    if (p >= a.nprob || (a.nprob_dev && p >= *a.nprob_dev)) return;
-    const ColiProb pr = uniform_prob(a.prob[p]);
-    const int m0 = mt * COLI_GM_ROWS;
-    const int nrows = min(COLI_GM_ROWS, pr.nrows - m0);
+    int p = 0, mt = item;
+    if (a.prob) {
+        const int tag = a.mt_list[item];
+        p = tag >> 16;
+        mt = tag & 0xffff;
+        if (p >= a.nprob || (a.nprob_dev && p >= *a.nprob_dev)) return;
+    }
+    const ColiProb pr = uniform_prob(a.prob ? a.prob[p] : a.prob0);
+    const int m0 = mt * COLI_GM_TILE;
+    const int nrows = min(COLI_GM_TILE, pr.nrows - m0);
     if (nrows <= 0) return;
+    const int Q0 = split * a.qps, nq = min(a.nq, Q0 + a.qps) - Q0;   // this workgroup's quads
+
+    const bool use_lo = *a.haslo >= a.lo_gen;   // >=: stays correct under graph replay
+    const int nm = (nrows + 15) >> 4;           // live 16-row subtiles
+    // the ring is written behind the compiler's back: let it escape, so the
+    // "memory" clobbers of the waits below force fresh reads (plain loads: no
+    // read moves across a wait or barrier, and the compiler may batch the
+    // reads of one step)
+    asm volatile("" ::"v"(lds) : "memory");
+
+    // Value(s) of row bl of the tile, output row 16 k + lane % 16 of the block
+    // (DUAL: v, u its gate and up), E the row's exponent: stored scaled back
+    // by 2^E, or with a K split as this split's raw partials. The exponents
+    // come through LDS with the first DMAs: loaded here they were a chain of
+    // one memory round trip a row (16384 rows of K 1024, 2048 outputs: 248 ->
+    // 210 us).
+    auto store = [&](int bl, int k, int E, float v, float u) {
+        if (bl >= nrows) return;
+        const int orow = pr.out_row0 + m0 + bl;
+        if (a.splits > 1) {
+            float *pp = a.partial + ((size_t)split * a.part_rows + orow) * a.rb_per_prob * (COLI_GM_BLOCK_TILES * 16) +
+                        (size_t)rb * (COLI_GM_BLOCK_TILES * 16) + (DUAL ? 32 : 16) * k + (lane & 15);
+            pp[0] = v;
+            if constexpr (DUAL) pp[16] = u;
+            return;
+        }
+        const int o = (rb * (COLI_GM_BLOCK_TILES / (DUAL ? 2 : 1)) + k) * 16 + (lane & 15);
+        if (o >= a.O) return;
+        float *y = a.out + (size_t)orow * a.ldo + o;
+        if constexpr (DUAL) *y = swiglu_out(ldexpf(v, E), ldexpf(u, E), a.swiglu_limit);
+        else *y = ldexpf(v, E);
+    };
+
+    if (nm > G::kMt) {
+        // tall tile: tile k of the block (DUAL: a wave's tiles 4 i .. 4 i + 3 =
+        // gate, gate, up, up of the block's row tiles 2 i, 2 i + 1); past the
+        // matrix its last row tile is read
+        auto tile_of = [&](int k, const uint8_t *&w, const uint8_t *&sc) {
+            const int r = min(DUAL ? rb * 8 + 2 * (k >> 2) + (k & 1) : rb * 16 + k, a.nrt - 1);
+            const bool second = DUAL && (k & 2);
+            const size_t t0 = (size_t)r * a.nq + Q0;
+            w = (const uint8_t *)(second ? pr.w1 : pr.w0) + t0 * COLI_TILE_BYTES;
+            sc = (const uint8_t *)(second ? pr.s1 : pr.s0) + t0 * SG::kBytes;
+        };
+        using T = GtGeom<KIND>;
+        const uint8_t *wt[2], *sp, *unused;
+        tile_of(wave, wt[0], unused);
+        tile_of(wave + 8, wt[1], unused);
+        // 1 KiB scale DMA wave % kScInst of the quad: lane l fetches 16 B of
+        // tile (16 / kScInst) (wave % kScInst) + l / (kBytes / 16)
+        constexpr int SL = SG::kBytes / 16;
+        tile_of((wave % T::kScInst) * (COLI_GM_BLOCK_TILES / T::kScInst) + lane / SL, unused, sp);
+        sp += (lane % SL) * 16;
+        // this lane's row and 16 B of the activation DMAs: row 16 wave + 8 k +
+        // l / 8, its eight 16 B pieces of a half quad stored XORed
+        uint32_t xo[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int r = 8 * k + (lane >> 3), br = pr.xrow_off + m0 + min(16 * wave + r, nrows - 1);
+            const int fr = a.xrows ? a.xrows[br] : br;
+            xo[k] = (uint32_t)fr * (uint32_t)a.xstride + 128 * Q0 + 8 * ((lane & 7) ^ tall_key(r));
+            // the row's exponent, once per lane of the row
+            __builtin_amdgcn_global_load_lds((const void *)(a.xexp + fr),
+                                             (lds_void *)(lds + GtGeom<KIND>::kExp + (2 * wave + k) * 256), 4, 0, 0);
+        }
+        const int *const es = (const int *)(lds + GtGeom<KIND>::kExp);
+        auto put = [&](int bl, int k, float v, float u) {
+            const int E = es[(bl >> 3) * 64 + (bl & 7) * 8];
+            if constexpr (DUAL) {
+                store(bl, 2 * (k >> 2) + (k & 1), E, v, u);
+            } else {
+                store(bl, k, E, v, 0.0f);
+                store(bl, k + 2, E, u, 0.0f);
+            }
+        };
+        // the second row half of a tile of up to 96 rows has one row block
+        auto go = [&](auto lo_tag, auto fold_tag) {
+            constexpr bool LO = decltype(lo_tag)::value, FOLD = decltype(fold_tag)::value;
+            if (nm <= 6 && wave >= 4)
+                gemm_tall<KIND, LO, FOLD, 1>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, lane, wave, put);
+            else
+                gemm_tall<KIND, LO, FOLD, 2>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, lane, wave, put);
+        };
+        auto by_fold = [&](auto lo_tag) {
+            if constexpr (KIND == COLI_KIND_FP4) {
+                if (a.fold) go(lo_tag, std::true_type{});
+                else go(lo_tag, std::false_type{});
+            } else {
+                go(lo_tag, std::false_type{});
+            }
+        };
+        if (use_lo) by_fold(std::true_type{});
+        else by_fold(std::false_type{});
+        return;
+    }
 
     int rt[R];
     bool live[R];
@@ -115,31 +481,30 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         const uint8_t *sc = (const uint8_t *)(second ? pr.s1 : pr.s0);
         // a dead tile re-reads tile (0, q) of the problem: the count of loads
         // stays fixed and no address is hammered by every quad
-        const size_t t0 = live[r] ? (size_t)rt[r] * a.nq : 0;
+        const size_t t0 = (live[r] ? (size_t)rt[r] * a.nq : 0) + Q0;
         wr[r] = w + t0 * COLI_TILE_BYTES;
         sr[r] = sc + t0 * SG::kBytes;
     }
-    const bool use_lo = *a.haslo >= a.lo_gen;   // >=: stays correct under graph replay
-    const int nm = (nrows + 15) >> 4;           // live 16-row subtiles
 
     // Activation chunks of this wave: c = wave + W k (m = c / 4, j = c % 4);
     // lane l fetches row 16 m + (l & 15) (clamped to the tile's last row),
     // columns 32 j + 8 (l >> 4) .. + 7.
     constexpr int CPW = G::kChunks / W;   // chunks per wave and stage half
     static_assert(G::kChunks % W == 0 && W % 4 == 0, "chunks must spread evenly over the waves");
-    int xoff[CPW];
+    uint32_t xoff[CPW];
 #pragma unroll
     for (int k = 0; k < CPW; k++) {
         const int r = min(16 * ((wave + W * k) >> 2) + (lane & 15), nrows - 1);
         const int br = pr.xrow_off + m0 + r;
         const int fr = a.xrows ? a.xrows[br] : br;
-        xoff[k] = fr * a.xstride + 32 * (wave & 3) + 8 * (lane >> 4);
+        xoff[k] = (uint32_t)fr * (uint32_t)a.xstride + 128 * Q0 + 32 * (wave & 3) + 8 * (lane >> 4);
     }
-    // the ring is written behind the compiler's back: let it escape, so the
-    // "memory" clobbers of the waits below force fresh reads (plain loads: no
-    // read moves across a wait or barrier, and the compiler may batch the
-    // reads of one step)
-    asm volatile("" ::"v"(lds) : "memory");
+    // the rows' exponents: wave w < 4 fetches subtile w's, four copies
+    if (wave < G::kMt) {
+        const int br = pr.xrow_off + m0 + min(16 * wave + (lane & 15), nrows - 1);
+        __builtin_amdgcn_global_load_lds((const void *)(a.xexp + (a.xrows ? a.xrows[br] : br)),
+                                         (lds_void *)(lds + G::kLds + wave * 256), 4, 0, 0);
+    }
 
     floatx4 acc[R][G::kMt];
 #pragma unroll
@@ -264,7 +629,6 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         // younger stages may stay in flight), barrier (every wave's chunks of
         // stage q have landed, and every wave is done with quad q - 1, whose
         // slot the next issue reuses), issue stage q + PD - 1, compute quad q.
-        const int nq = a.nq;
 #pragma unroll
         for (int i = 0; i < PD - 1; i++)
             if (i < nq) issue(i, i);
@@ -316,44 +680,69 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         by_lo(std::false_type{});
     }
 
-    // epilogue: batch row m0 + 16 m + 4 (lane / 16) + i, output row rt * 16 + lane % 16
+    const int *const es = (const int *)(lds + G::kLds);
 #pragma unroll
     for (int m = 0; m < G::kMt; m++) {
         if (m >= nm) break;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int bl = m * 16 + 4 * (lane >> 4) + i;
-            if (bl >= nrows) continue;
-            const int br = pr.xrow_off + m0 + bl;
-            const int E = a.xexp[a.xrows ? a.xrows[br] : br];
-            float *orow = a.out + (size_t)(pr.out_row0 + m0 + bl) * a.ldo;
+        for (int i = 0; i < 4; i++)
 #pragma unroll
             for (int t = 0; t < RT; t++) {
+                const int bl = m * 16 + 4 * (lane >> 4) + i;
                 const int r = DUAL ? 2 * t : t;   // the gate (DUAL) or the plain tile of row tile t
-                if (!live[r]) continue;
-                const int o = rt[r] * 16 + (lane & 15);
-                if (o >= a.O) continue;
-                if constexpr (DUAL)
-                    orow[o] = swiglu_out(ldexpf(acc[r][m][i], E), ldexpf(acc[r + 1][m][i], E), a.swiglu_limit);
-                else orow[o] = ldexpf(acc[r][m][i], E);
+                store(bl, wave * RT + t, es[m * 64 + (bl & 15)], acc[r][m][i], DUAL ? acc[DUAL ? r + 1 : r][m][i] : 0.0f);
             }
-        }
     }
+}
+
+// Sum of a K-split GEMM's partials in split order, then the GEMM's epilogue
+// (2^E of the row, SwiGLU of the gate / up columns). One thread per output
+// value; output row o of the matrix lies in block o / (16 T), column 16 c + o %
+// 16 with c its tile in the block (DUAL: tiles 2i, 2i + 1).
+template <bool DUAL>
+__global__ __launch_bounds__(256) void coli_gemm_reduce(const float *__restrict__ part, int splits, int rows, int rb,
+                                                        int O, const int *__restrict__ xexp, float *__restrict__ out,
+                                                        int ldo, float swiglu_limit) {
+    constexpr int RPB = COLI_GM_BLOCK_TILES * 16 / (DUAL ? 2 : 1);   // output rows of a block
+    const int o = blockIdx.x * 256 + threadIdx.x, r = blockIdx.y;
+    if (o >= O) return;
+    const int ld = rb * COLI_GM_BLOCK_TILES * 16;
+    const int c = DUAL ? (o / RPB) * 256 + 32 * ((o % RPB) >> 4) + (o & 15) : o;
+    float v = 0.0f, u = 0.0f;
+    for (int s = 0; s < splits; s++) {
+        const float *p = part + ((size_t)s * rows + r) * ld + c;
+        v += p[0];
+        if constexpr (DUAL) u += p[16];
+    }
+    const int E = xexp[r];
+    out[(size_t)r * ldo + o] = DUAL ? swiglu_out(ldexpf(v, E), ldexpf(u, E), swiglu_limit) : ldexpf(v, E);
 }
 
 template <int KIND>
 static hipError_t launch_gemm_kind(const ColiGemmArgs &a, bool dual, hipStream_t st) {
-    const dim3 grid((unsigned)a.n_mt * a.rb_per_prob), block(64 * COLI_GM_W);
-    const size_t shm = GmGeom<KIND>::kLds;
+    const dim3 grid((unsigned)a.n_mt * a.splits * a.rb_per_prob), block(64 * COLI_GM_W);
+    const size_t shm = GmGeom<KIND>::kLds + 1024;   // the short tiles' exponents after the ring
     if (dual) hipLaunchKernelGGL((coli_gemm_tiles<KIND, true>), grid, block, shm, st, a);
     else hipLaunchKernelGGL((coli_gemm_tiles<KIND, false>), grid, block, shm, st, a);
+    if (a.splits > 1) {
+        const dim3 rg((a.O + 255) / 256, a.part_rows);
+        if (dual)
+            hipLaunchKernelGGL(coli_gemm_reduce<true>, rg, dim3(256), 0, st, a.partial, a.splits, a.part_rows,
+                               a.rb_per_prob, a.O, a.xexp, a.out, a.ldo, a.swiglu_limit);
+        else
+            hipLaunchKernelGGL(coli_gemm_reduce<false>, rg, dim3(256), 0, st, a.partial, a.splits, a.part_rows,
+                               a.rb_per_prob, a.O, a.xexp, a.out, a.ldo, 0.0f);
+    }
     return hipGetLastError();
 }
 
 // rb_per_prob must cover the output rows: 8 (dual) or 16 row tiles per block.
 extern "C" hipError_t coli_launch_gemm(int kind, int dual, const ColiGemmArgs *a, hipStream_t st) {
     if (a->n_mt <= 0 || a->rb_per_prob <= 0) return hipSuccess;
-    if ((long)a->n_mt * a->rb_per_prob > 0x7fffffffL || !a->mt_list) return hipErrorInvalidValue;
+    if ((long)a->n_mt * a->splits * a->rb_per_prob > 0x7fffffffL || (a->prob && !a->mt_list)) return hipErrorInvalidValue;
+    // a K split: output rows [0, part_rows) in fragment-row order, at most 65535 of them
+    if (a->splits < 1 || a->qps < 1 || (a->splits > 1 && (!a->partial || a->xrows || a->part_rows < 1 || a->part_rows > 65535)))
+        return hipErrorInvalidValue;
     switch (kind) {
     case COLI_KIND_I4_H: return launch_gemm_kind<COLI_KIND_I4_H>(*a, dual != 0, st);
     case COLI_KIND_I4_F: return launch_gemm_kind<COLI_KIND_I4_F>(*a, dual != 0, st);

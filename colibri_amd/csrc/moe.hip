@@ -17,7 +17,7 @@
 // (an expert's rows start at the sum of the earlier experts' counts), so h
 // and y hold S*K (+S) rows whatever the batch. Up to COLI_GEMM_MIN_ROWS rows
 // the experts run the tiled GEMV; beyond, the grouped GEMM over a device-built
-// list of 64-row tiles. Every stage is stream-ordered on the device; nothing
+// list of 128-row tiles. Every stage is stream-ordered on the device; nothing
 // returns to the host between stages, and no stage allocates once the layer
 // has run at a given S.
 #include "coli_hip_host.h"
@@ -63,7 +63,7 @@ struct ColiHipMoe {
 // are placed by an LDS counter (the placement of a row inside its list does
 // not change any result: every row is computed on its own, and the combine
 // addresses rows through slotrow).
-// Also emits the GEMM work list (expert << 16 | 64-row tile) in union order.
+// Also emits the GEMM work list (expert << 16 | row tile of `tile` rows) in union order.
 // ---------------------------------------------------------------------------
 // The body runs on any block size; sm: (7 E + 5) ints of LDS. idx / keff may
 // point to LDS.
@@ -71,7 +71,8 @@ __device__ __forceinline__ void moe_union_body(const int *idx, const int *keff, 
                                                const ColiProb *__restrict__ tab, ColiProb *__restrict__ pdual,
                                                ColiProb *__restrict__ pdown, int *__restrict__ uniq,
                                                int *__restrict__ xrows, int *__restrict__ slotrow,
-                                               int *__restrict__ mt, int *__restrict__ state, int *sm) {
+                                               int *__restrict__ mt, int *__restrict__ state, int *sm,
+                                               int tile = COLI_GM_TILE) {
     // first [E] | cnt [E] | cur [E] | rank [E] | order [E + 1] | off [E + 2] | toff [E + 2]
     int *first = sm, *cnt = first + E, *cur = cnt + E, *rank = cur + E, *order = rank + E, *off = order + E + 1,
         *toff = off + E + 2;
@@ -143,7 +144,7 @@ __device__ __forceinline__ void moe_union_body(const int *idx, const int *keff, 
             int c = 0, tl = 0;
             if (j < np) {
                 c = order[j] == E ? S : cnt[order[j]];
-                tl = (c + COLI_GM_ROWS - 1) / COLI_GM_ROWS;
+                tl = (c + tile - 1) / tile;
             }
             int xc = c, xt = tl;
 #pragma unroll
@@ -197,7 +198,7 @@ __device__ __forceinline__ void moe_union_body(const int *idx, const int *keff, 
         d.out_row0 = dn.out_row0 = off[j];
         pdual[j] = d;
         pdown[j] = dn;
-        for (int q = 0; q * COLI_GM_ROWS < c; q++) mt[toff[j] + q] = j << 16 | q;
+        for (int q = 0; q * tile < c; q++) mt[toff[j] + q] = j << 16 | q;
     }
     if (threadIdx.x == 0) {
         state[0] = np;
@@ -269,7 +270,7 @@ __device__ __forceinline__ void moe_union_wave(const int *idx, const int *keff, 
         d.out_row0 = dn.out_row0 = off;
         pdual[rank] = d;
         pdown[rank] = dn;
-        mt[rank] = rank << 16;   // one 64-row tile per expert (total <= S <= 64)
+        mt[rank] = rank << 16;   // one row tile per expert (total <= S <= 64)
     }
     const int np = nu + (has_shared ? 1 : 0);
     if (has_shared) {
@@ -298,9 +299,9 @@ __global__ __launch_bounds__(1024) void coli_moe_union(const int *__restrict__ i
                                                        const ColiProb *__restrict__ tab, ColiProb *__restrict__ pdual,
                                                        ColiProb *__restrict__ pdown, int *__restrict__ uniq,
                                                        int *__restrict__ xrows, int *__restrict__ slotrow,
-                                                       int *__restrict__ mt, int *__restrict__ state) {
+                                                       int *__restrict__ mt, int *__restrict__ state, int tile) {
     extern __shared__ int sm[];
-    moe_union_body(idx, keff, S, K, E, has_shared, tab, pdual, pdown, uniq, xrows, slotrow, mt, state, sm);
+    moe_union_body(idx, keff, S, K, E, has_shared, tab, pdual, pdown, uniq, xrows, slotrow, mt, state, sm, tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -1120,8 +1121,8 @@ extern "C" int coli_hip_moe_create(ColiHipMoe **out, int device, const ColiHipMo
 // Upper bounds of one forward of S rows.
 static int moe_problems(const ColiHipMoeConfig &c, int S) { return std::min(c.E, S * c.K) + (c.has_shared ? 1 : 0); }
 static int moe_rows(const ColiHipMoeConfig &c, int S) { return S * c.K + (c.has_shared ? S : 0); }
-static int moe_tiles(const ColiHipMoeConfig &c, int S) {
-    return (moe_rows(c, S) + COLI_GM_ROWS - 1) / COLI_GM_ROWS + moe_problems(c, S);
+static int moe_tiles(const ColiHipMoeConfig &c, int S, int tile) {
+    return (moe_rows(c, S) + tile - 1) / tile + moe_problems(c, S);
 }
 
 // Per-forward buffers for up to S rows (allocated once per growth of S).
@@ -1140,7 +1141,7 @@ static int moe_reserve(DevCtx *ctx, ColiHipMoe *m, int S) {
         }
     const size_t sizes[] = {(size_t)coli_router_chunks(c.D) * S * c.E * 4, (size_t)S * c.K * 4,
                             (size_t)rows * c.I * 4, (size_t)rows * c.D * 4, (size_t)S * c.K * 4, (size_t)S * 4, 16,
-                            (size_t)c.E * 4, (size_t)rows * 4, (size_t)S * c.K * 4, (size_t)moe_tiles(c, S) * 4,
+                            (size_t)c.E * 4, (size_t)rows * 4, (size_t)S * c.K * 4, (size_t)moe_tiles(c, S, COLI_GM_ROWS) * 4,
                             (size_t)P * sizeof(ColiProb), (size_t)P * sizeof(ColiProb)};
     for (int i = 0; i < 13; i++)
         if (!hip_check(hipMalloc(bufs[i], sizes[i]), "moe buffers")) return 0;
@@ -1368,6 +1369,7 @@ static int moe_forward_impl(ColiHipMoe *m, DevCtx *ctx, const float *x_dev, floa
     hipStream_t st = ctx->stream;
     // many-row MXFP4 layers run the block-scaled MFMA GEMM on e4m3 pieces
     const bool gemm = S > COLI_GEMM_MIN_ROWS, mx = gemm && m->kind == COLI_KIND_FP4 && mx_gemm_enabled();
+    const int tile = mx ? COLI_GM_ROWS : COLI_GM_TILE;
     // 1. activation fragments, 2-3. router
     if (!(mx ? make_frags8(ctx, fx, x_dev, c.D, S, c.D) : make_frags(ctx, fx, x_dev, c.D, S, c.D, int4))) return 0;
     const int nrt_i = (c.I + 15) / 16, nrt_d = (c.D + 15) / 16;
@@ -1421,7 +1423,7 @@ static int moe_forward_impl(ColiHipMoe *m, DevCtx *ctx, const float *x_dev, floa
         // 4. union
         const size_t ush = (size_t)(7 * c.E + 5) * sizeof(int);
         hipLaunchKernelGGL(coli_moe_union, dim3(1), dim3(1024), ush, st, m->idx, m->keff, S, c.K, c.E, c.has_shared,
-                           m->tab, m->pdual, m->pdown, m->uniq, m->xrows, m->slotrow, m->mt, m->state);
+                           m->tab, m->pdual, m->pdown, m->uniq, m->xrows, m->slotrow, m->mt, m->state, tile);
         if (!hip_check(hipGetLastError(), "moe union")) return 0;
     }
     // 5. gate/up + SwiGLU over the union, 6. hidden fragments, 7. down
@@ -1431,7 +1433,7 @@ static int moe_forward_impl(ColiHipMoe *m, DevCtx *ctx, const float *x_dev, floa
     for (size_t i = 0; fold && i < m->mats.size(); i++) fold = m->mats[i]->e8_fold != 0;
     if (gateup_done) {
     } else if (gemm) {
-        if (!run_gemm(ctx, m->kind, true, m->pdual, P, m->state, m->mt, m->state + 3, moe_tiles(c, S), nrt_i, nq_d,
+        if (!run_gemm(ctx, m->kind, true, m->pdual, P, m->state, m->mt, m->state + 3, moe_tiles(c, S, tile), nrt_i, nq_d,
                       c.I, fx, m->xrows, m->h, c.I, c.swiglu_limit, fold))
             return 0;
     } else if (S == 1 && dual1_enabled() && launch_dual1(m, st, x_dev, nrt_i, nq_d, P, shared_overlap)) {
@@ -1482,7 +1484,7 @@ static int moe_forward_impl(ColiHipMoe *m, DevCtx *ctx, const float *x_dev, floa
              : make_frags(ctx, fh, m->h, c.I, rows, c.I, int4, nullptr, m->state + 1)))
         return 0;
     if (gemm) {
-        if (!run_gemm(ctx, m->kind, false, m->pdown, P, m->state, m->mt, m->state + 3, moe_tiles(c, S), nrt_d, nq_i,
+        if (!run_gemm(ctx, m->kind, false, m->pdown, P, m->state, m->mt, m->state + 3, moe_tiles(c, S, tile), nrt_d, nq_i,
                       c.D, fh, nullptr, m->y, c.D, 0.0f, fold))
             return 0;
     } else if (!run_gemv(ctx, m->kind, false, m->pdown, P, m->state, nrt_d, nq_i, c.D, S, fh, nullptr, m->y, c.D,
