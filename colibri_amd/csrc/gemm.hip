@@ -17,17 +17,17 @@
 //    wave's weight tiles and their scales (private to the wave), and the
 //    quad's activation fragments of the tile's rows (fp16 hi + lo of x * 2^-E,
 //    built by coli_prep_frag; shared by the workgroup, each wave fetching a
-//    fixed number of the 1 KiB chunks). No load of the loop writes a
+//    number of the 1 KiB chunks that depends on the live subtiles). No load of the loop writes a
 //    register, so the compiler inserts no wait of its own: the loop waits with
 //    exact s_waitcnt vmcnt(N) for its oldest stage and synchronizes with a
 //    bare s_barrier (the fence of __syncthreads() would drain the ring). The
 //    activations ride in the same ring as the weights, as deep: loads retire
 //    in order, so a shallower activation ring would retire the weights with it;
-//  * the chunks are laid out in the MFMA A-operand order (lane l of a DMA
-//    fetches the 16 B lane l of the MFMA reads), so the reads are free of bank
-//    conflicts; chunks of dead 16-row subtiles read the tile's last row (one
-//    cache line) into a trash slot, which keeps the count of loads per stage
-//    fixed;
+//  * an activation chunk is 4 rows x 256 B, whole cache lines (16 rows x 64 B, and
+//    as many DMAs for dead subtiles as for live ones, before: the 384-expert
+//    MXFP4 layer at 512 rows 1086 -> 1051 us),
+//    its 16 B pieces XOR-swizzled so the operand reads are free of bank
+//    conflicts;
 //  * the loop is specialized per (lo parts present, folded scales, live
 //    16-row subtiles NM): the stage holds only NM subtiles' activations, so
 //    short tiles (the common prefill case of a few rows per expert) stream
@@ -64,7 +64,6 @@
 template <int KIND>
 struct GmGeom {
     static constexpr int kMt = COLI_GM_ROWS / 16;                 // 16-row subtiles per tile
-    static constexpr int kChunks = 4 * kMt;                        // 1 KiB activation chunks per stage half
     static constexpr int kW = COLI_GM_W, kR = COLI_GM_BLOCK_TILES / COLI_GM_W;   // waves, tiles per wave
     static constexpr int scale_inst(int rn) { return (rn + ScaleGeom<KIND>::kPerInst - 1) / ScaleGeom<KIND>::kPerInst; }
     static constexpr int wslot(int rn) { return rn * COLI_TILE_BYTES + scale_inst(rn) * 256; }
@@ -486,19 +485,6 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         sr[r] = sc + t0 * SG::kBytes;
     }
 
-    // Activation chunks of this wave: c = wave + W k (m = c / 4, j = c % 4);
-    // lane l fetches row 16 m + (l & 15) (clamped to the tile's last row),
-    // columns 32 j + 8 (l >> 4) .. + 7.
-    constexpr int CPW = G::kChunks / W;   // chunks per wave and stage half
-    static_assert(G::kChunks % W == 0 && W % 4 == 0, "chunks must spread evenly over the waves");
-    uint32_t xoff[CPW];
-#pragma unroll
-    for (int k = 0; k < CPW; k++) {
-        const int r = min(16 * ((wave + W * k) >> 2) + (lane & 15), nrows - 1);
-        const int br = pr.xrow_off + m0 + r;
-        const int fr = a.xrows ? a.xrows[br] : br;
-        xoff[k] = (uint32_t)fr * (uint32_t)a.xstride + 128 * Q0 + 32 * (wave & 3) + 8 * (lane >> 4);
-    }
     // the rows' exponents: wave w < 4 fetches subtile w's, four copies
     if (wave < G::kMt) {
         const int br = pr.xrow_off + m0 + min(16 * wave + (lane & 15), nrows - 1);
@@ -524,7 +510,26 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         constexpr int SI = G::scale_inst(RN);
         constexpr int WS = G::wslot(RN);
         static_assert(PD >= 3, "the ring needs three stages");
-        constexpr int L = RN + SI + (LO ? 2 : 1) * CPW;   // DMA instructions per wave and stage
+        // Activation chunks of a stage: 4 rows x 256 B (whole cache lines),
+        // the NM subtiles' hi chunks, then lo. Wave w fetches chunks w, w + 8,
+        // ...: only as many DMAs as the live subtiles need (their count
+        // depends on NM alone); a chunk past the end reads row 0 of the tile
+        // into the trash slot. The sixteen 16 B pieces of a row are stored
+        // XORed with row % 16, so the sixteen lanes of one k-slice read
+        // sixteen different slots.
+        constexpr int NCH = 4 * NM * (LO ? 2 : 1), CPW = (NCH + W - 1) / W;
+        constexpr int L = RN + SI + CPW;   // DMA instructions per wave and stage
+        uint32_t xoff[CPW];
+#pragma unroll
+        for (int k = 0; k < CPW; k++) {
+            const int c = (wave + W * k) % (4 * NM), r = 4 * c + (lane >> 4);   // row of the tile
+            const int br = pr.xrow_off + m0 + min(wave + W * k < NCH ? r : 0, nrows - 1);
+            const int fr = a.xrows ? a.xrows[br] : br;
+            xoff[k] = (uint32_t)fr * (uint32_t)a.xstride + 128 * Q0 + 8 * ((lane & 15) ^ (r & 15));
+        }
+        int xrd[4];   // the lane's 16 B of group j in a subtile
+#pragma unroll
+        for (int j = 0; j < 4; j++) xrd[j] = (lane & 15) * 256 + 16 * ((4 * j + (lane >> 4)) ^ (lane & 15));
         uint8_t *const ring = lds + G::kRing;
         uint8_t *const wring = ring + PD * ACT + wave * PD * WS;
         auto issue = [&](int q, int slot) {
@@ -546,14 +551,10 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
             uint8_t *xs = ring + slot * ACT;
 #pragma unroll
             for (int k = 0; k < CPW; k++) {
-                const size_t o = (size_t)xoff[k] + (size_t)q * 128;
                 const int c = wave + W * k;
-                // chunks of dead subtiles read the clamped last row into the trash slot
-                uint8_t *dst = c < 4 * NM ? xs + c * 1024 : lds + G::kTrash;
-                __builtin_amdgcn_global_load_lds((const void *)(a.xhi + o), (lds_void *)dst, 16, 0, 0);
-                if constexpr (LO)
-                    __builtin_amdgcn_global_load_lds((const void *)(a.xlo + o),
-                                                     (lds_void *)(c < 4 * NM ? dst + LOFF : dst), 16, 0, 0);
+                const _Float16 *src = LO && c >= 4 * NM ? a.xlo : a.xhi;   // (lo chunks follow the hi ones in the stage)
+                __builtin_amdgcn_global_load_lds((const void *)(src + (size_t)xoff[k] + (size_t)q * 128),
+                                                 (lds_void *)(c < NCH ? xs + c * 1024 : lds + G::kTrash), 16, 0, 0);
             }
         };
         auto compute = [&](int slot) {
@@ -580,7 +581,7 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
                 half8v xh[NM], xl[NM];
 #pragma unroll
                 for (int m = 0; m < NM; m++) {
-                    const uint8_t *fo = xs + (m * 4 + j) * 1024 + lane * 16;
+                    const uint8_t *fo = xs + m * 4096 + xrd[j];
                     xh[m] = *(const half8v *)fo;
                     if constexpr (LO) xl[m] = *(const half8v *)(fo + LOFF);
                 }
