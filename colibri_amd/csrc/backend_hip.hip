@@ -200,6 +200,7 @@ extern "C" void coli_cuda_shutdown(void) {
         if (ctx->host_prob.h) (void)hipHostFree(ctx->host_prob.h);
         if (ctx->host_small.h) (void)hipHostFree(ctx->host_small.h);
         if (ctx->ev_ok) (void)hipEventDestroy(ctx->ev_done);
+        for (int e = 0; e < ctx->n_piece_ev; e++) (void)hipEventDestroy(ctx->ev_piece[e]);
         if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
         *ctx = DevCtx();
     }

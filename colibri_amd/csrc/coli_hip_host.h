@@ -26,6 +26,11 @@
 #define COLI_NA_BYTES ((size_t)8 << 20)
 #define COLI_NA_PART_BYTES (COLI_NA_BYTES - COLI_NA_OFF_PART)
 
+// Many host rows cross PCIe in pieces of this size (at most COLI_PIECES,
+// larger then), the host's copy of one beside the transfer of another.
+#define COLI_PIECE_BYTES ((size_t)512 << 10)
+#define COLI_PIECES 32
+
 struct DevBuf {
     void *p = nullptr;
     size_t cap = 0;
@@ -85,6 +90,9 @@ struct DevCtx {
     // coli_hip_pipe_gemm_noalloc), looked up at init; null if unavailable
     uint8_t *scratch = nullptr;
     FragSet na_frag;                   // views into scratch (no allocations)
+    // completion of the pieces of a download (see download_piped)
+    hipEvent_t ev_piece[COLI_PIECES] = {};
+    int n_piece_ev = 0;
     int group_pending = 0;
     hipEvent_t ev_done = nullptr;
     int ev_ok = 0;

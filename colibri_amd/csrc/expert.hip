@@ -693,26 +693,83 @@ static double now_ms() {
     return std::chrono::duration<double, std::milli>(clk::now().time_since_epoch()).count();
 }
 
-// Stage host x -> device, run, device y -> pinned host_y (not yet synchronized).
+// Host rows to the device through the pinned staging buffer: piece i is on
+// its way while the host copies piece i + 1 into the buffer (one copy of all of
+// it, then one transfer, before: 256 rows of 5120 in and out through an
+// expert, 553 -> 467 us with download_piped; the host's copy takes 70 us and
+// the transfer 102 us each way). Pieces of 512 KiB through copy kernels
+// measured best (DMA-engine copies 1 MiB 501 us, 512 KiB 563).
+static size_t piece_bytes(size_t bytes) {
+    const size_t p = std::max(COLI_PIECE_BYTES, (bytes + COLI_PIECES - 1) / COLI_PIECES);
+    return (p + 4095) & ~(size_t)4095;
+}
+
+static int upload_piped(DevCtx *ctx, void *dst, const PinBuf &pin, const void *src, size_t bytes, bool kcopy) {
+    const size_t piece = piece_bytes(bytes);
+    for (size_t o = 0; o < bytes; o += piece) {
+        const size_t n = std::min(piece, bytes - o);
+        std::memcpy((char *)pin.h + o, (const char *)src + o, n);
+        if (!hip_check(kcopy ? coli_launch_copy_f32((float *)((char *)dst + o), (const float *)((char *)pin.d + o), n / 4,
+                                                    ctx->stream)
+                             : hipMemcpyAsync((char *)dst + o, (char *)pin.h + o, n, hipMemcpyHostToDevice, ctx->stream),
+                       "input upload"))
+            return 0;
+    }
+    return 1;
+}
+
+// Device rows to the host: the pieces are queued behind the work on the
+// stream and each is copied out of the pinned buffer when it has arrived,
+// while the next one is on its way. Nothing is written to dst before the work
+// that computes the rows has ended without an error.
+static int download_piped(DevCtx *ctx, void *dst, const PinBuf &pin, const void *src, size_t bytes, bool kcopy) {
+    const size_t piece = piece_bytes(bytes);
+    const int n = (int)((bytes + piece - 1) / piece);
+    for (; ctx->n_piece_ev < n; ctx->n_piece_ev++)
+        if (!hip_check(hipEventCreateWithFlags(&ctx->ev_piece[ctx->n_piece_ev], hipEventDisableTiming), "piece event"))
+            return 0;
+    for (int i = 0; i < n; i++) {
+        const size_t o = i * piece;
+        const size_t nb = std::min(piece, bytes - o);
+        if (!hip_check(kcopy ? coli_launch_copy_f32((float *)((char *)pin.d + o), (const float *)((const char *)src + o),
+                                                    nb / 4, ctx->stream)
+                             : hipMemcpyAsync((char *)pin.h + o, (const char *)src + o, nb, hipMemcpyDeviceToHost,
+                                              ctx->stream),
+                       "output download") ||
+            !hip_check(hipEventRecord(ctx->ev_piece[i], ctx->stream), "piece event"))
+            return 0;
+    }
+    for (int i = 0; i < n; i++) {
+        const size_t o = i * piece;
+        if (!hip_check(hipEventSynchronize(ctx->ev_piece[i]), "output synchronize")) return 0;
+        std::memcpy((char *)dst + o, (const char *)pin.h + o, std::min(piece, bytes - o));
+    }
+    return hip_check(hipStreamSynchronize(ctx->stream), "output synchronize");
+}
+
+// Stage host x -> device, run, device y -> pinned host_y (not yet
+// synchronized). Rows of more than a piece each way, with y_host given: out to
+// y_host, synchronized (*done).
 static int group_stage_and_run(DevCtx *ctx, std::vector<Member> &mem, int count, int total, int D, int I,
-                               const float *x, hipEvent_t *ev) {
+                               const float *x, hipEvent_t *ev, float *y_host = nullptr, bool *done = nullptr) {
     size_t xb = (size_t)total * D * sizeof(float);
     if (!reserve(ctx, &ctx->x, xb, 0) || !reserve(ctx, &ctx->y, xb, 0) ||
         !reserve_pinned(ctx, &ctx->host_x, xb) ||
         !reserve_pinned(ctx, &ctx->host_y, xb))
         return 0;
     if (!hip_check(hipStreamSynchronize(ctx->stream), "group staging")) return 0;
-    std::memcpy(ctx->host_x.h, x, xb);
+    const bool piped = y_host && xb > ((size_t)1 << 20);
+    if (!piped) std::memcpy(ctx->host_x.h, x, xb);
     if (ev) (void)hipEventRecord(ev[0], ctx->stream);
     // Decode-sized groups cross PCIe in copy kernels that read / write the
     // pinned buffers through their device addresses (measured: the sync group
-    // call at decode 47 -> 39 us against DMA-engine copies). Above 1 MiB each
-    // way (prefill-sized groups) the DMA engines' hipMemcpyAsync is used, as
-    // always with COLI_HIP_KCOPY=0.
+    // call at decode 47 -> 39 us against DMA-engine copies); above 1 MiB each
+    // way (prefill-sized groups) in pieces. COLI_HIP_KCOPY=0: hipMemcpyAsync.
     const char *kc = std::getenv("COLI_HIP_KCOPY");
-    const bool kcopy = !(kc && kc[0] == '0') && xb <= ((size_t)1 << 20);
+    const bool kernels = !(kc && kc[0] == '0'), kcopy = kernels && xb <= ((size_t)1 << 20);
     void *hx_dev = ctx->host_x.d, *hy_dev = ctx->host_y.d;
-    if (kcopy ? !hip_check(coli_launch_copy_f32((float *)ctx->x.p, (const float *)hx_dev, xb / 4, ctx->stream),
+    if (piped ? !upload_piped(ctx, ctx->x.p, ctx->host_x, x, xb, kernels)
+        : kcopy ? !hip_check(coli_launch_copy_f32((float *)ctx->x.p, (const float *)hx_dev, xb / 4, ctx->stream),
                         "group input upload")
               : !hip_check(hipMemcpyAsync(ctx->x.p, ctx->host_x.h, xb, hipMemcpyHostToDevice, ctx->stream),
                         "group input upload"))
@@ -722,6 +779,15 @@ static int group_stage_and_run(DevCtx *ctx, std::vector<Member> &mem, int count,
     if (!run_expert_group(ctx, mem.data(), count, total, D, I, (float *)ctx->y.p, (const float *)ctx->x.p, true))
         return 0;
     if (ev) (void)hipEventRecord(ev[2], ctx->stream);
+    if (piped) {
+        const int ok = download_piped(ctx, y_host, ctx->host_y, ctx->y.p, xb, kernels);
+        if (ev) {
+            (void)hipEventRecord(ev[3], ctx->stream);
+            (void)hipEventSynchronize(ev[3]);
+        }
+        *done = ok != 0;
+        return ok;
+    }
     if (kcopy ? !hip_check(coli_launch_copy_f32((float *)hy_dev, (const float *)ctx->y.p, xb / 4, ctx->stream),
                         "group output download")
               : !hip_check(hipMemcpyAsync(ctx->host_y.h, ctx->y.p, xb, hipMemcpyDeviceToHost, ctx->stream),
@@ -749,8 +815,9 @@ extern "C" int coli_cuda_expert_group(ColiCudaTensor *const *gates, ColiCudaTens
                 profile = 0;
                 break;
             }
-    int ok = group_stage_and_run(ctx, mem, count, total, D, I, x, profile ? ev : nullptr) &&
-             hip_check(hipStreamSynchronize(ctx->stream), "expert group synchronize");
+    bool done = false;
+    int ok = group_stage_and_run(ctx, mem, count, total, D, I, x, profile ? ev : nullptr, y, &done) &&
+             (done || hip_check(hipStreamSynchronize(ctx->stream), "expert group synchronize"));
     double a = 0, b = 0, c = 0;
     if (profile) {
         float fa = 0, fb = 0, fc = 0;
@@ -763,7 +830,7 @@ extern "C" int coli_cuda_expert_group(ColiCudaTensor *const *gates, ColiCudaTens
         for (int i = 0; i < 4; i++) (void)hipEventDestroy(ev[i]);
     }
     if (!ok) return 0;
-    std::memcpy(y, ctx->host_y.h, (size_t)total * D * sizeof(float));
+    if (!done) std::memcpy(y, ctx->host_y.h, (size_t)total * D * sizeof(float));
     note_group(ctx, count, total, a, b, c);
     return 1;
 }
@@ -803,10 +870,11 @@ extern "C" int coli_cuda_expert_mlp(ColiCudaTensor *gate, ColiCudaTensor *up, Co
     int total, D, I;
     DevCtx *ctx = collect_members(g, u, d, rows, 1, mem, &total, &D, &I);
     if (!ctx || ctx->group_pending) return 0;
-    if (!group_stage_and_run(ctx, mem, 1, total, D, I, x, nullptr) ||
-        !hip_check(hipStreamSynchronize(ctx->stream), "expert mlp synchronize"))
+    bool done = false;
+    if (!group_stage_and_run(ctx, mem, 1, total, D, I, x, nullptr, y, &done) ||
+        (!done && !hip_check(hipStreamSynchronize(ctx->stream), "expert mlp synchronize")))
         return 0;
-    std::memcpy(y, ctx->host_y.h, (size_t)total * D * sizeof(float));
+    if (!done) std::memcpy(y, ctx->host_y.h, (size_t)total * D * sizeof(float));
     return 1;
 }
 
