@@ -55,7 +55,8 @@ struct ColiHipMoe {
 };
 
 // ---------------------------------------------------------------------------
-// union + descriptor build, one 1024-thread block.
+// union + descriptor build, one block (decode and small batches;
+// coli_moe_union below for more rows).
 // Selection i = (t, kk) in row-major order is live when kk < keff[t] and its
 // expert is in range. The union lists the experts in first-seen order: an
 // expert's rank is the number of experts whose first live selection comes
@@ -63,7 +64,7 @@ struct ColiHipMoe {
 // are placed by an LDS counter (the placement of a row inside its list does
 // not change any result: every row is computed on its own, and the combine
 // addresses rows through slotrow).
-// Also emits the GEMM work list (expert << 16 | row tile of `tile` rows) in union order.
+// Also emits the GEMM work list (expert << 16 | row tile of COLI_GM_TILE rows) in union order.
 // ---------------------------------------------------------------------------
 // The body runs on any block size; sm: (7 E + 5) ints of LDS. idx / keff may
 // point to LDS.
@@ -71,8 +72,8 @@ __device__ __forceinline__ void moe_union_body(const int *idx, const int *keff, 
                                                const ColiProb *__restrict__ tab, ColiProb *__restrict__ pdual,
                                                ColiProb *__restrict__ pdown, int *__restrict__ uniq,
                                                int *__restrict__ xrows, int *__restrict__ slotrow,
-                                               int *__restrict__ mt, int *__restrict__ state, int *sm,
-                                               int tile = COLI_GM_TILE) {
+                                               int *__restrict__ mt, int *__restrict__ state, int *sm) {
+    constexpr int tile = COLI_GM_TILE;   // (decode and small batches: at most 64 rows an expert, one tile either way)
     // first [E] | cnt [E] | cur [E] | rank [E] | order [E + 1] | off [E + 2] | toff [E + 2]
     int *first = sm, *cnt = first + E, *cur = cnt + E, *rank = cur + E, *order = rank + E, *off = order + E + 1,
         *toff = off + E + 2;
@@ -294,14 +295,128 @@ __device__ __forceinline__ void moe_union_wave(const int *idx, const int *keff, 
     }
 }
 
+// The union of up to COLI_MOE_MAX_SEL selections (prefill) by one 1024-thread
+// block: moe_union_body with a thread's selections (at most 16) held in
+// registers over its passes, all requested in one memory round trip (read
+// again pass by pass they were up to 48 dependent ones), and the experts'
+// ranks counted from their first positions (no scan over the selections).
+// Bound by latency: 2048 x 8 selections of 64 experts 36 -> 18-25 us, 512 x 8 of
+// 384 14 -> 12-20 us (the int4 layer of 64 experts at 2048 rows 642 -> 622 us).
 __global__ __launch_bounds__(1024) void coli_moe_union(const int *__restrict__ idx, const int *__restrict__ keff,
                                                        int S, int K, int E, int has_shared,
                                                        const ColiProb *__restrict__ tab, ColiProb *__restrict__ pdual,
                                                        ColiProb *__restrict__ pdown, int *__restrict__ uniq,
                                                        int *__restrict__ xrows, int *__restrict__ slotrow,
                                                        int *__restrict__ mt, int *__restrict__ state, int tile) {
-    extern __shared__ int sm[];
-    moe_union_body(idx, keff, S, K, E, has_shared, tab, pdual, pdown, uniq, xrows, slotrow, mt, state, sm, tile);
+    // first [E, padded to 4] | cnt [E] | off [E] by expert | order [E]
+    extern __shared__ __attribute__((aligned(16))) int sm_union[];
+    const int E4 = (E + 3) & ~3;
+    int *first = sm_union, *cnt = first + E4, *off = cnt + E, *order = off + E;
+    __shared__ int s_nu, s_ws[16], s_wt[16];
+    constexpr int NV = COLI_MOE_MAX_SEL / 1024;
+    const int n = S * K, tid = threadIdx.x, w = tid >> 6, ln = tid & 63;
+    int ev[NV], kv[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+        const int i = tid + 1024 * v;
+        ev[v] = i < n ? idx[i] : -1;
+        kv[v] = i < n ? keff[i / K] : 0;
+    }
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+        if (1024 * v >= n) continue;   // (block-uniform; ev is -1 there)
+        const int i = tid + 1024 * v;
+        if (ev[v] < 0 || ev[v] >= E || i - i / K * K >= kv[v]) ev[v] = -1;
+    }
+    for (int e = tid; e < E4; e += 1024) {
+        first[e] = 0x7fffffff;
+        if (e < E) cnt[e] = 0;
+    }
+    if (tid == 0) s_nu = 0;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < NV; v++)
+        if (ev[v] >= 0) {
+            atomicMin(first + ev[v], tid + 1024 * v);
+            atomicAdd(cnt + ev[v], 1);
+        }
+    __syncthreads();
+    // rank of an expert in first-seen order: how many were seen before it
+    // (E <= 1024: one thread an expert)
+    int rank = -1;
+    if (tid < E && first[tid] != 0x7fffffff) {
+        const int f = first[tid];
+        rank = 0;
+#pragma unroll 8
+        for (int k = 0; k < E4; k += 4) {
+            const int4 q = *(const int4 *)(first + k);
+            rank += (q.x < f) + (q.y < f) + (q.z < f) + (q.w < f);
+        }
+        order[rank] = tid;
+    }
+    const unsigned long long seen = __builtin_amdgcn_ballot_w64(rank >= 0);
+    if (ln == 0) atomicAdd(&s_nu, __popcll(seen));
+    __syncthreads();
+    const int nu = s_nu, np = nu + (has_shared ? 1 : 0);
+    // packed row and tile offsets in union order: problem tid's exclusive
+    // prefix (np <= 1025: thread 0 takes the shared expert's after the scan)
+    const int e_of = tid < nu ? order[tid] : -1;
+    const int c = e_of >= 0 ? cnt[e_of] : 0, tl = (c + tile - 1) / tile;
+    int xc = c, xt = tl;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int yc = __shfl_up(xc, o), yt = __shfl_up(xt, o);
+        if (ln >= o) {
+            xc += yc;
+            xt += yt;
+        }
+    }
+    if (ln == 63) {
+        s_ws[w] = xc;
+        s_wt[w] = xt;
+    }
+    __syncthreads();
+    int pc = 0, pt = 0, rows = 0, tiles = 0;
+    for (int v = 0; v < 16; v++) {
+        pc += v < w ? s_ws[v] : 0;
+        pt += v < w ? s_wt[v] : 0;
+        rows += s_ws[v];
+        tiles += s_wt[v];
+    }
+    const int my_off = pc + xc - c, my_toff = pt + xt - tl;
+    if (e_of >= 0) off[e_of] = my_off;
+    auto emit = [&](int j, int e, int cn, int o, int to) {
+        ColiProb d = tab[2 * e], dn = tab[2 * e + 1];
+        d.nrows = dn.nrows = cn;
+        d.xrow_off = dn.xrow_off = o;
+        d.out_row0 = dn.out_row0 = o;
+        pdual[j] = d;
+        pdown[j] = dn;
+        for (int q = 0; q * tile < cn; q++) mt[to + q] = j << 16 | q;
+    };
+    if (e_of >= 0) {
+        uniq[tid] = e_of;
+        emit(tid, e_of, c, my_off, my_toff);
+    }
+    if (has_shared) {
+        if (tid == 0) emit(nu, E, S, rows, tiles);
+        for (int t = tid; t < S; t += 1024) xrows[rows + t] = t;
+    }
+    __syncthreads();
+    // the experts' rows, placed by their offset's counter
+#pragma unroll
+    for (int v = 0; v < NV; v++)
+        if (ev[v] >= 0) {
+            const int i = tid + 1024 * v, row = atomicAdd(off + ev[v], 1);
+            xrows[row] = i / K;
+            slotrow[i] = row;
+        }
+    if (tid == 0) {
+        state[0] = np;
+        state[1] = rows + (has_shared ? S : 0);
+        state[2] = nu;
+        state[3] = tiles + (has_shared ? (S + tile - 1) / tile : 0);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1421,7 +1536,7 @@ static int moe_forward_impl(ColiHipMoe *m, DevCtx *ctx, const float *x_dev, floa
                             "moe router select"))
             return 0;
         // 4. union
-        const size_t ush = (size_t)(7 * c.E + 5) * sizeof(int);
+        const size_t ush = (size_t)(4 * c.E + 3) * sizeof(int);
         hipLaunchKernelGGL(coli_moe_union, dim3(1), dim3(1024), ush, st, m->idx, m->keff, S, c.K, c.E, c.has_shared,
                            m->tab, m->pdual, m->pdown, m->uniq, m->xrows, m->slotrow, m->mt, m->state, tile);
         if (!hip_check(hipGetLastError(), "moe union")) return 0;
