@@ -936,9 +936,15 @@ static int gemm_rows(DevCtx *ctx, ColiCudaTensor *t, const void *sc, int set, fl
 // to 14336 x 4096). Crossovers measured (GEMV / GEMM): 4096 x 14336 17 rows 41
 // / 31 us; 14336 x 4096 32 rows 29 / 27; 4096 x 4096 128 rows 30 / 35, 192
 // rows 42 / 40; 2048 x 7168 128 rows 28 / 37, 192 rows 46 / 40; 512 x 2048
-// 1024 rows 28 / 39.
+// 1024 rows 28 / 39. COLI_HIP_GEMV=dma|tiles pins the GEMV here too, =gemm the
+// GEMM (tuning and tests).
 static bool dense_on_gemm(const DevCtx *ctx, const ColiCudaTensor *t, int S) {
-    if (S <= 16 || S > 65535) return S > 16;
+    if (S <= 16) return false;
+    if (const char *f = std::getenv("COLI_HIP_GEMV")) {
+        if (std::strcmp(f, "gemm") == 0) return true;
+        if (std::strcmp(f, "dma") == 0 || std::strcmp(f, "tiles") == 0) return false;
+    }
+    if (S > 65535) return true;
     const int rb = (t->nrt + COLI_GM_BLOCK_TILES - 1) / COLI_GM_BLOCK_TILES;
     int splits;
     const double gemm = gemm_plan(ctx, (S + COLI_GM_TILE - 1) / COLI_GM_TILE, rb, t->nq, std::min(S, COLI_GM_TILE), S,

@@ -45,39 +45,73 @@ def test_grouped_gemm_row_tiles(session, fmt, lo, e8, rows):
         o += r
 
 
-@pytest.mark.parametrize("fmt,half,O,I,S", [
-    (4, True, 4096, 14336, 17),     # one short tile, K split
-    (4, False, 2064, 7184, 200),    # f32 scales, tall tiles, K split, ragged block and columns
-    (7, True, 4112, 4112, 193),     # MXFP4, a short tile of one row behind a tall one
-    (4, True, 14336, 1040, 129),    # blocks enough for the chip
-])
-def test_dense_rows_on_the_gemm(session, fmt, half, O, I, S):
-    """pipe_gemm of more rows than a GEMV batch tile, where the GEMM is the
-    faster: the same product, also on a second call of fewer rows."""
-    rng = np.random.default_rng(O + S)
+def upload_dense(session, rng, fmt, half, O, I):
+    """(handle, group size, dequantized weights, oracle product)."""
     if fmt == 7:
         q, sc = rand_mxfp4(rng, O, I)
-        h, deq = session.upload_mxfp4(q, sc, I, O), deq_mxfp4(q, sc, I)
-    else:
-        q, sc = rand_i4(rng, O, I, 32, fp16_scales=half)
-        h, deq = session.upload(q, sc, 4, I, O, 32), deq_i4(q, sc, I, 32)
+        return session.upload_mxfp4(q, sc, I, O), 0, deq_mxfp4(q, sc, I), lambda x: cref.matmul_mxfp4(x, q, sc, O, I)
+    q, sc = rand_i4(rng, O, I, 32, fp16_scales=half)
+    return (session.upload(q, sc, 4, I, O, 32), 32, deq_i4(q, sc, I, 32),
+            lambda x: cref.matmul_i4_grouped(x, q, sc, O, I, 32))
+
+
+@pytest.mark.parametrize("fmt,half,O,I,S", [
+    (4, True, 4096, 14336, 18),     # one short tile, K split
+    (4, False, 2064, 7184, 200),    # f32 scales, tall tiles, K split, ragged block and columns
+    (7, True, 4112, 4112, 194),     # MXFP4, a short tile of two rows behind a tall one
+    (4, True, 14336, 1040, 130),    # blocks enough for the chip
+    (7, False, 528, 128, 100),      # one quad of K: every prefetch past the end is clamped
+    (4, False, 528, 256, 97),       # two
+])
+def test_dense_rows_on_the_gemm(session, monkeypatch, fmt, half, O, I, S):
+    """Dense matrices of more rows than a GEMV batch tile, pinned to the GEMM:
+    the same product, also on a second call of one row less."""
+    monkeypatch.setenv("COLI_HIP_GEMV", "gemm")
+    rng = np.random.default_rng(O + S)
+    h, gs, deq, product = upload_dense(session, rng, fmt, half, O, I)
     x = rng.standard_normal((S, I)).astype(np.float32)
     try:
-        got = {s: session.matmul(h, x[:s], fmt, I, O, 0 if fmt == 7 else 32) for s in (S, S - 1)}
+        got = {s: session.matmul(h, x[:s], fmt, I, O, gs) for s in (S, S - 1)}
     finally:
         session.free(h)
-    ref = cref.matmul_mxfp4(x, q, sc, O, I) if fmt == 7 else cref.matmul_i4_grouped(x, q, sc, O, I, 32)
+    ref = product(x)
     mag = magnitude(x, deq)
     for s, y in got.items():
         assert rel_err(y, ref[:s], mag[:s]).max() <= TOL
         assert (np.abs(y.astype(np.float64) - ref[:s]) / mag[:s]).max() <= 2 * err_bound(I)   # ref rounds as well
 
 
-@pytest.mark.parametrize("S", [24, 130])
-def test_idot_rows_on_the_gemm_bitwise(session, S):
-    """fmt=2 with int8 activations for many rows: every sum is an exact
-    integer, so the K split changes nothing and the result is the
+@pytest.mark.parametrize("fmt,O,I,S,gemm", [(4, 4096, 14336, 48, True), (4, 14336, 4096, 512, True),
+                                            (7, 4096, 4096, 320, True), (4, 512, 2048, 512, False),
+                                            (4, 4096, 14336, 16, False)])
+def test_dense_kernel_pin(session, monkeypatch, fmt, O, I, S, gemm):
+    """COLI_HIP_GEMV pins dense matrices of more than 16 rows to either
+    kernel (their sums round in another order, so the results differ in
+    bits), and the rule without it takes the one expected for shapes well
+    inside its side."""
+    rng = np.random.default_rng(3 * O + S)
+    h, gs, _, _ = upload_dense(session, rng, fmt, True, O, I)
+    x = rng.standard_normal((S, I)).astype(np.float32)
+    got = {}
+    try:
+        for pin in ("tiles", "gemm", None):
+            if pin:
+                monkeypatch.setenv("COLI_HIP_GEMV", pin)
+            else:
+                monkeypatch.delenv("COLI_HIP_GEMV", raising=False)
+            got[pin] = session.matmul(h, x, fmt, I, O, gs)
+    finally:
+        session.free(h)
+    assert np.array_equal(got["tiles"], got["gemm"]) == (S <= 16)
+    assert np.array_equal(got[None], got["gemm" if gemm else "tiles"])
+
+
+@pytest.mark.parametrize("S", [24, 48, 130])
+def test_idot_rows_on_the_gemm_bitwise(session, monkeypatch, S):
+    """fmt=2 with int8 activations for many rows on the GEMM: every sum is an
+    exact integer, so the K split changes nothing and the result is the
     reference's."""
+    monkeypatch.setenv("COLI_HIP_GEMV", "gemm")
     rng = np.random.default_rng(S)
     O, I = 4096, 8192
     q, sc = rand_i4(rng, O, I, 0)
