@@ -184,7 +184,7 @@ extern "C" void coli_cuda_shutdown(void) {
         DevCtx *ctx = &g_ctx[i];
         if (!bind_ctx(ctx)) continue;
         (void)hipStreamSynchronize(ctx->stream);
-        DevBuf *bufs[] = {&ctx->x, &ctx->h, &ctx->y, &ctx->g, &ctx->u, &ctx->partial,
+        DevBuf *bufs[] = {&ctx->x, &ctx->h, &ctx->y, &ctx->g, &ctx->u, &ctx->partial, &ctx->sums,
                           &ctx->prob, &ctx->stage_w, &ctx->stage_s, &ctx->qdq, &ctx->flags,
                           &ctx->rslot, &ctx->rw, &ctx->tmp_tiles, &ctx->tmp_scales, &ctx->zeros,
                           &ctx->split_cnt, &ctx->idot_y, &ctx->idot_sx};

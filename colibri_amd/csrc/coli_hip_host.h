@@ -79,7 +79,7 @@ struct DevCtx {
     hipStream_t stream = nullptr;
     size_t tensor_count = 0, tensor_bytes = 0;
     // grow-only scratch
-    DevBuf x, h, y, g, u, partial, prob, zeros, stage_w, stage_s, qdq, flags;
+    DevBuf x, h, y, g, u, partial, sums, prob, zeros, stage_w, stage_s, qdq, flags;
     DevBuf rslot, rw, tmp_tiles, tmp_scales, split_cnt, idot_y, idot_sx;
     FragSet frag[4];                   // 0/1: inputs (int4 / fp4 order), 2/3: hidden rows
     int dense_set[2] = {0, 1};         // set the next coli_hip_gemm_run_dev reads, per order (gemm_prep)

@@ -131,6 +131,7 @@ struct ColiGemvArgs {
 #define COLI_GM_ROWS 64     // rows of a short tile (and of the block-scaled variant's tiles)
 #endif
 #define COLI_GM_TILE 128    // rows of a work item of coli_gemm_tiles
+#define COLI_GM_SUMS (COLI_GM_TILE * COLI_GM_BLOCK_TILES * 16)   // outputs of a workgroup
 
 struct ColiGemmArgs {
     const ColiProb *prob;     // device descriptors; null: the single problem prob0 (item i = its row tile i)
@@ -154,6 +155,8 @@ struct ColiGemmArgs {
     float swiglu_limit;       // > 0: DeepSeek-V4 clamped SwiGLU in the DUAL epilogue
     int fold;                 // MXFP4, every matrix e8_fold: scales folded into the unpacked operand
     int splits, qps;          // K split: quads per split; 1: none
+    int segq;                 // quads summed in one running sum (plain matrices; >= qps: all)
+    float *sums;              // [workgroup][(qps - 1) / segq][COLI_GM_SUMS]: a tall tile's sums so far (segq < qps)
     float *partial;           // [split][part_rows][rb_per_prob * 256] raw sums (splits > 1)
     int part_rows;            // output rows of the call (splits > 1: fragment row r is output row r)
 };

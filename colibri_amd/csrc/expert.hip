@@ -407,6 +407,22 @@ static double gemm_plan(const DevCtx *ctx, long items, int rb, int nq, int tile,
     return best;
 }
 
+// Quads of K that the GEMV sums in one running sum for S rows of a dense
+// matrix: its waves (at least four for a single matrix) and K splits each take
+// a share. The GEMM keeps to it for the matrices that dense_on_gemm sends
+// there: one f32 chain over all of K rounds once a group, and its error grows
+// with the square root of its length (512 x 14336 x 4096, distance from the
+// 64-bit product: GEMV 1.30e-7; GEMM 2.14e-7 as one chain, 1.62e-7 as two,
+// 1.30e-7 as four, the GEMV's number). For the same reason MXFP4 scales are
+// not folded there: folded, the running sum is the MFMA's accumulator and
+// rounds twice a group, hi and lo product (40 x 14336 x 4096: GEMV 1.16e-7,
+// folded with half the chain 1.42e-7).
+static int dense_chain(const DevCtx *ctx, int nrt, int nq, int S) {
+    const GemvLaunchPlan g = plan_gemv(ctx, 1, (S + 15) / 16, nrt, nq, false, S);
+    const int W = std::max(4, g.W);
+    return std::max(1, (g.qps + W - 1) / W);
+}
+
 // Grouped GEMM over problems of many rows (see gemm.hip); mt_list_dev holds
 // n_mt entries (problem << 16 | row tile), problem indices relative to
 // probs_dev. inline_prob: the single problem instead of descriptors and list.
@@ -477,7 +493,7 @@ int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     a.out = out;
     a.ldo = ldo;
     a.swiglu_limit = swiglu_limit;
-    a.fold = fold && kind == COLI_KIND_FP4;
+    a.fold = fold && kind == COLI_KIND_FP4 && !inline_prob;   // (see dense_chain)
     a.splits = 1;
     if (split_rows > 0 && split_rows <= 65535) {
         const long cols = (long)a.rb_per_prob * COLI_GM_BLOCK_TILES * 16;
@@ -490,7 +506,34 @@ int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     }
     a.qps = (nq + a.splits - 1) / a.splits;
     a.splits = (nq + a.qps - 1) / a.qps;
-    return hip_check(coli_launch_gemm(kind, dual ? 1 : 0, &a, ctx->stream), "gemm launch");
+    // (int8 activations: every sum is an exact integer, whatever its order)
+    a.segq = a.qps;
+    if (inline_prob && !f.nolo) {
+        const int chain = dense_chain(ctx, nrt, nq, inline_prob->nrows);
+        const int segs = (a.qps + chain - 1) / chain;
+        a.segq = (a.qps + segs - 1) / segs;
+    }
+    // Tall tiles keep their sums so far in scratch memory, as large as the
+    // result for every running sum but the last: beyond 512 MiB the row tiles
+    // go in several launches (one after the other on the stream).
+    int step = n_mt;
+    if (a.segq < a.qps && inline_prob->nrows > COLI_GM_ROWS) {
+        const size_t item = (size_t)a.splits * a.rb_per_prob * ((a.qps - 1) / a.segq) * COLI_GM_SUMS * sizeof(float);
+        if (a.splits == 1) step = (int)std::max((size_t)1, std::min((size_t)n_mt, ((size_t)512 << 20) / item));
+        if (!reserve(ctx, &ctx->sums, step * item, 0)) return 0;
+        a.sums = (float *)ctx->sums.p;
+    }
+    for (int i = 0; i < n_mt; i += step) {
+        ColiGemmArgs b = a;
+        if (step < n_mt) {
+            b.n_mt = std::min(step, n_mt - i);
+            b.prob0.nrows -= i * COLI_GM_TILE;
+            b.prob0.xrow_off += i * COLI_GM_TILE;
+            b.prob0.out_row0 += i * COLI_GM_TILE;
+        }
+        if (!hip_check(coli_launch_gemm(kind, dual ? 1 : 0, &b, ctx->stream), "gemm launch")) return 0;
+    }
+    return 1;
 }
 
 int frag_set_of(int kind, bool hidden) {

@@ -121,6 +121,19 @@ __device__ __forceinline__ int tall_off(int lane, int g, int t) {
 // rows x 64 B ran at half the rate). store(row, tile of the block, gate or
 // plain value, value of the tile after it) takes the results.
 //
+// Folded MXFP4 scales (a.fold) are not used here: with two 32x32x16 MFMAs a
+// product, accumulating inside them would round twice as often as the short
+// tiles' one 16x16x32 does (300 x 8192 x 4096, 64 groups to a running sum:
+// 3.4e-7 from the 64-bit product against 2.0e-7 so).
+//
+// SEG: segq quads at most go into one running sum (see dense_chain,
+// expert.hip). The sums so far are written to this wave's part of a scratch
+// buffer, one set after another (nothing waits for the stores), and added at
+// the end: a second set of accumulators does not fit the registers (spilled
+// inside the loop), and adding to the first set in memory every time waits for
+// it behind the ring's DMAs (the 512-row feed-forward of 4096 x 14336 int4:
+// 397 us as one chain, 480 us with the sums added in memory, SEGTIME so).
+//
 // The loop is a sequence of steps, one per (group, row block, column block):
 // the step's 2 (4 with lo parts) MFMAs beside the work that needs no result of
 // theirs: the LDS reads of the next fragments, the scaling of the previous
@@ -133,10 +146,10 @@ __device__ __forceinline__ int tall_off(int lane, int g, int t) {
 // on the GEMV kernel, 155 us with the same tiles scheduled by the compiler,
 // 119-139 us here (1.0 PFLOP/s of MFMA work; 1.2 MXFP4; a bf16 library product
 // of 8192^3 reaches 1.4 on the card).
-template <int KIND, bool LO, bool FOLD, int NB, typename Store>
+template <int KIND, bool LO, int NB, bool SEG, typename Store>
 __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, const uint8_t *wt1, const uint8_t *sp,
                                           const _Float16 *xhi, const _Float16 *xlo, uint32_t xo0, uint32_t xo1, int nq,
-                                          int lane, int wave, Store store) {
+                                          int segq, float *sums, int lane, int wave, Store store) {
     using T = GtGeom<KIND>;
     using SG = ScaleGeom<KIND>;
     constexpr int PD = T::pd(LO), NW = T::nw(LO), ACT = T::act(LO), WS = T::kWSlot;
@@ -198,8 +211,7 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
     };
     auto unpack = [&](int n, int t, int j) {
         if (t == 0) scl[j & 1][n] = sc[n].get(j);
-        if constexpr (FOLD) bw[j & 1][n][t] = unpack_fp4_scaled(w[n][t][j], scl[j & 1][n]);
-        else bw[j & 1][n][t] = unpack_b<KIND>(w[n][t][j]);
+        bw[j & 1][n][t] = unpack_b<KIND>(w[n][t][j]);
     };
     const int xofs[2][2] = {{tall_off(lane, 0, 0), tall_off(lane, 0, 1)}, {tall_off(lane, 1, 0), tall_off(lane, 1, 1)}};
     auto load_x = [&](int p, const uint8_t *xs, int g, int b) {   // group g (0, 1) of the half quad, row block b
@@ -213,12 +225,10 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
     auto scale = [&](auto pt, auto bt, auto nt, auto jt) {   // products d[p] of blocks (b, n), group parity jp
         constexpr int p = decltype(pt)::value, b = decltype(bt)::value, n = decltype(nt)::value;
         constexpr int jp = decltype(jt)::value;
-        if constexpr (!FOLD) {
-            floatx16 v = acc[b][n];
+        floatx16 v = acc[b][n];
 #pragma unroll
-            for (int i = 0; i < 16; i++) v[i] = fmaf(d[p][i], scl[jp][n], v[i]);
-            acc[b][n] = v;
-        }
+        for (int i = 0; i < 16; i++) v[i] = fmaf(d[p][i], scl[jp][n], v[i]);
+        acc[b][n] = v;
     };
     auto wait_lds = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
     auto barrier = [&]() {
@@ -278,7 +288,6 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
         // after the ring's synchronization
         if constexpr (half_end ? n == 1 : n == 0) load_x(p ^ 1, aslot(as), (lastb ? j + 1 : j) & 1, lastb ? 0 : b + 1);
         floatx16 z = {};
-        if constexpr (FOLD) z = acc[b][n];
 #pragma unroll
         for (int t = 0; t < 2; t++) z = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[p][t], bw[j & 1][n][t], z, 0, 0, 0);
         if constexpr (LO) {
@@ -286,8 +295,7 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
             for (int t = 0; t < 2; t++)
                 z = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[p][t], bw[j & 1][n][t], z, 0, 0, 0);
         }
-        if constexpr (FOLD) acc[b][n] = z;
-        else d[dp] = z;
+        d[dp] = z;
         // scale the previous step's products (n - 1 of this row block, or n =
         // 1 of the one before)
         constexpr int pb = n == 1 ? b : (b == 0 ? NB - 1 : b - 1), pj = n == 1 || b > 0 ? j : j + 3;
@@ -305,7 +313,7 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
         }
         // an MFMA first: the wait for this step's operands then comes before
         // the next fragments' reads are queued behind them
-        constexpr int NM = LO ? 4 : 2, NV = FOLD ? 6 / NM : (16 + 12 * (4 / NS) + NM - 1) / NM;
+        constexpr int NM = LO ? 4 : 2, NV = (16 + 12 * (4 / NS) + NM - 1) / NM;
 #pragma unroll
         for (int k = 0; k < NM; k++) {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
@@ -324,17 +332,56 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
             step(c, jt, C1{}, C1{});
         }
     };
-    for (int c = 0; c < nq; c++) {
+    auto quad = [&](int c) {
         group(c, std::integral_constant<int, 0>{});
         group(c, std::integral_constant<int, 1>{});
         group(c, std::integral_constant<int, 2>{});
         group(c, std::integral_constant<int, 3>{});
         wn1 = wn1 == NW - 1 ? 0 : wn1 + 1;
+    };
+    if constexpr (!SEG) {
+        for (int c = 0; c < nq; c++) quad(c);
+    } else {
+        // (the last step's products, not scaled yet, open the next sum)
+        for (int c = 0;;) {
+            for (const int ce = min(nq, c + segq); c < ce; c++) quad(c);
+            if (c >= nq) break;
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int n = 0; n < 2; n++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        floatx4 v;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            v[i] = acc[b][n][4 * k + i];
+                            acc[b][n][4 * k + i] = 0.0f;
+                        }
+                        *(floatx4 *)(sums + (b * 8 + n * 4 + k) * 256 + lane * 4) = v;
+                    }
+            sums += COLI_GM_SUMS;
+        }
     }
     scale(std::integral_constant<int, 1>{}, std::integral_constant<int, NB - 1>{}, std::integral_constant<int, 1>{},
           std::integral_constant<int, 1>{});
     // the last DMAs write this workgroup's LDS: none may outlive it
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (SEG) {
+        for (int c = segq; c < nq; c += segq) {
+            sums -= COLI_GM_SUMS;
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int n = 0; n < 2; n++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const floatx4 v = *(const floatx4 *)(sums + (b * 8 + n * 4 + k) * 256 + lane * 4);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[b][n][4 * k + i] += v[i];
+                    }
+        }
+    }
     // lane l, register i: row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32
 #pragma unroll
     for (int b = 0; b < NB; b++)
@@ -343,7 +390,8 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
             store(wm * 64 + b * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3), 4 * wn + l16, acc[b][0][i], acc[b][1][i]);
 }
 
-template <int KIND, bool DUAL>
+// SEG: a.segq quads at most in one running sum (plain matrices).
+template <int KIND, bool DUAL, bool SEG>
 __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a) {
     using G = GmGeom<KIND>;
     using SG = ScaleGeom<KIND>;
@@ -446,24 +494,21 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
                 store(bl, k + 2, E, u, 0.0f);
             }
         };
+        float *sums = nullptr;
+        if constexpr (SEG)
+            sums = a.sums + (size_t)blockIdx.x * ((a.qps - 1) / a.segq) * COLI_GM_SUMS + wave * (COLI_GM_SUMS / COLI_GM_W);
         // the second row half of a tile of up to 96 rows has one row block
-        auto go = [&](auto lo_tag, auto fold_tag) {
-            constexpr bool LO = decltype(lo_tag)::value, FOLD = decltype(fold_tag)::value;
+        auto go = [&](auto lo_tag) {
+            constexpr bool LO = decltype(lo_tag)::value;
             if (nm <= 6 && wave >= 4)
-                gemm_tall<KIND, LO, FOLD, 1>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, lane, wave, put);
+                gemm_tall<KIND, LO, 1, SEG>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, a.segq, sums, lane,
+                                            wave, put);
             else
-                gemm_tall<KIND, LO, FOLD, 2>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, lane, wave, put);
+                gemm_tall<KIND, LO, 2, SEG>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, a.segq, sums, lane,
+                                            wave, put);
         };
-        auto by_fold = [&](auto lo_tag) {
-            if constexpr (KIND == COLI_KIND_FP4) {
-                if (a.fold) go(lo_tag, std::true_type{});
-                else go(lo_tag, std::false_type{});
-            } else {
-                go(lo_tag, std::false_type{});
-            }
-        };
-        if (use_lo) by_fold(std::true_type{});
-        else by_fold(std::false_type{});
+        if (use_lo) go(std::true_type{});
+        else go(std::false_type{});
         return;
     }
 
@@ -634,14 +679,40 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         for (int i = 0; i < PD - 1; i++)
             if (i < nq) issue(i, i);
         int slot = 0;
-        for (int q = 0; q < nq; q++) {
-            dma_wait_tail<L, PD>(min(PD - 2, nq - 1 - q));
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            if (q + PD - 1 < nq) issue(q + PD - 1, slot == 0 ? PD - 1 : slot - 1);
-            compute(slot);
-            slot = slot == PD - 1 ? 0 : slot + 1;
+        auto pass = [&](int q0, int q1) {
+            for (int q = q0; q < q1; q++) {
+                dma_wait_tail<L, PD>(min(PD - 2, nq - 1 - q));
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                if (q + PD - 1 < nq) issue(q + PD - 1, slot == 0 ? PD - 1 : slot - 1);
+                compute(slot);
+                slot = slot == PD - 1 ? 0 : slot + 1;
+            }
+        };
+        if constexpr (!SEG) {
+            pass(0, nq);
+        } else {
+            // at most segq quads in one running sum (see dense_chain, expert.hip)
+            floatx4 tot[RN][NM];
+#pragma unroll
+            for (int t = 0; t < RN; t++)
+#pragma unroll
+                for (int m = 0; m < NM; m++) tot[t][m] = (floatx4){0.f, 0.f, 0.f, 0.f};
+            for (int q = 0; q < nq; q += a.segq) {
+                pass(q, min(nq, q + a.segq));
+#pragma unroll
+                for (int t = 0; t < RN; t++)
+#pragma unroll
+                    for (int m = 0; m < NM; m++) {
+                        tot[t][m] += acc[RB + t][m];
+                        acc[RB + t][m] = (floatx4){0.f, 0.f, 0.f, 0.f};
+                    }
+            }
+#pragma unroll
+            for (int t = 0; t < RN; t++)
+#pragma unroll
+                for (int m = 0; m < NM; m++) acc[RB + t][m] = tot[t][m];
         }
     };
     // one specialization per (lo parts, folded scales, live subtiles); one
@@ -674,7 +745,7 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         if (use_lo) by_nm(std::true_type{}, fold_tag);
         else by_nm(std::false_type{}, fold_tag);
     };
-    if constexpr (KIND == COLI_KIND_FP4) {
+    if constexpr (KIND == COLI_KIND_FP4 && !SEG) {
         if (a.fold) by_lo(std::true_type{});
         else by_lo(std::false_type{});
     } else {
@@ -723,8 +794,9 @@ template <int KIND>
 static hipError_t launch_gemm_kind(const ColiGemmArgs &a, bool dual, hipStream_t st) {
     const dim3 grid((unsigned)a.n_mt * a.splits * a.rb_per_prob), block(64 * COLI_GM_W);
     const size_t shm = GmGeom<KIND>::kLds + 1024;   // the short tiles' exponents after the ring
-    if (dual) hipLaunchKernelGGL((coli_gemm_tiles<KIND, true>), grid, block, shm, st, a);
-    else hipLaunchKernelGGL((coli_gemm_tiles<KIND, false>), grid, block, shm, st, a);
+    if (dual) hipLaunchKernelGGL((coli_gemm_tiles<KIND, true, false>), grid, block, shm, st, a);
+    else if (a.segq < a.qps) hipLaunchKernelGGL((coli_gemm_tiles<KIND, false, true>), grid, block, shm, st, a);
+    else hipLaunchKernelGGL((coli_gemm_tiles<KIND, false, false>), grid, block, shm, st, a);
     if (a.splits > 1) {
         const dim3 rg((a.O + 255) / 256, a.part_rows);
         if (dual)
@@ -742,7 +814,7 @@ extern "C" hipError_t coli_launch_gemm(int kind, int dual, const ColiGemmArgs *a
     if (a->n_mt <= 0 || a->rb_per_prob <= 0) return hipSuccess;
     if ((long)a->n_mt * a->splits * a->rb_per_prob > 0x7fffffffL || (a->prob && !a->mt_list)) return hipErrorInvalidValue;
     // a K split: output rows [0, part_rows) in fragment-row order, at most 65535 of them
-    if (a->splits < 1 || a->qps < 1 || (a->splits > 1 && (!a->partial || a->xrows || a->part_rows < 1 || a->part_rows > 65535)))
+    if (a->splits < 1 || a->qps < 1 || a->segq < 1 || (a->segq < a->qps && (a->prob || (!a->sums && a->prob0.nrows > COLI_GM_ROWS))) || (a->splits > 1 && (!a->partial || a->xrows || a->part_rows < 1 || a->part_rows > 65535)))
         return hipErrorInvalidValue;
     switch (kind) {
     case COLI_KIND_I4_H: return launch_gemm_kind<COLI_KIND_I4_H>(*a, dual != 0, st);

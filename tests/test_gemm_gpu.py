@@ -124,3 +124,76 @@ def test_idot_rows_on_the_gemm_bitwise(session, monkeypatch, S):
     finally:
         session.free(h)
     assert np.array_equal(y, cref.matmul_i4_idot(x, q, sc, O, I))
+
+
+@pytest.mark.parametrize("fmt,half,O,I,S", [
+    (4, True, 14336, 4096, 512),    # unsplit tall tiles, two running sums
+    (4, False, 4112, 4112, 200),    # a K split, a short tile behind a tall one, ragged block and columns
+    (7, True, 8192, 4096, 300),     # MXFP4
+    (7, True, 14336, 4096, 40),     # MXFP4, a short tile
+    (4, True, 14336, 4096, 40),     # a short tile
+    (4, True, 14336, 7168, 128),    # several running sums a split
+])
+def test_dense_gemm_rounds_no_more_than_the_gemv(session, monkeypatch, fmt, half, O, I, S):
+    """The GEMM's distance from the 64-bit product (2-norm over the whole
+    result) is at most the GEMV's, whose waves each sum a share of K: as many
+    running sums bound the growth of the f32 rounding the same way. 3 %: both
+    norms are sums over at least 5e5 values' independent errors (0.2 %), and
+    a last running sum of another length."""
+    rng = np.random.default_rng(11 * O + S)
+    h, gs, deq, _ = upload_dense(session, rng, fmt, half, O, I)
+    x = rng.standard_normal((S, I)).astype(np.float32)
+    err = {}
+    try:
+        for pin in ("tiles", "gemm"):
+            monkeypatch.setenv("COLI_HIP_GEMV", pin)
+            got = session.matmul(h, x, fmt, I, O, gs)
+            if not err:
+                exact = x.astype(np.float64) @ deq.T.astype(np.float64)
+            err[pin] = np.linalg.norm(got - exact) / np.linalg.norm(exact)
+    finally:
+        session.free(h)
+    assert err["gemm"] <= 1.03 * err["tiles"], err
+
+
+def test_dense_gemm_row_tiles_in_several_launches(session, monkeypatch):
+    """More rows than the scratch memory for the running sums holds at once
+    (24 row tiles of this shape): each launch's rows land where they belong."""
+    rng = np.random.default_rng(60)
+    O, I, S = 14336, 4096, 3077
+    h, gs, _, _ = upload_dense(session, rng, 4, True, O, I)
+    x = rng.standard_normal((S, I)).astype(np.float32)
+    try:
+        monkeypatch.setenv("COLI_HIP_GEMV", "gemm")
+        y = session.matmul(h, x, 4, I, O, gs)
+        monkeypatch.setenv("COLI_HIP_GEMV", "tiles")
+        ref = session.matmul(h, x, 4, I, O, gs)
+    finally:
+        session.free(h)
+    d = np.linalg.norm(y - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert d.max() <= 1e-6   # (two results with 1.3e-7 of rounding each)
+
+
+def test_tall_mxfp4_tiles_round_no_more_than_short_ones(session):
+    """Eight members of 128 rows (tall tiles) against the same rows as sixteen
+    members of 64 (short tiles, whose folded scales accumulate in the MFMA):
+    the distance from the 64-bit result does not grow. Enough blocks that
+    gate/up runs without a K split."""
+    rng = np.random.default_rng(77)
+    D, I = 2048, 4096
+    layer = Layer(rng, 7, D, I, 1)
+    hs = layer.upload(session)
+    x = rng.standard_normal((1024, D)).astype(np.float32)
+    q, u, d = (deq_mxfp4(*layer.experts[0][i], K) for i, K in enumerate((D, D, I)))
+    a = x.astype(np.float64) @ q.T
+    exact = (a / (1 + np.exp(-a)) * (x.astype(np.float64) @ u.T)) @ d.T
+    err = {}
+    try:
+        for rows in (128, 64):
+            n = 1024 // rows
+            y = session.expert_group([hs[0][0]] * n, [hs[0][1]] * n, [hs[0][2]] * n, [rows] * n, x)
+            err[rows] = np.linalg.norm(y - exact) / np.linalg.norm(exact)
+    finally:
+        for t in hs[0]:
+            session.free(t)
+    assert err[128] <= 1.03 * err[64], err
