@@ -121,18 +121,13 @@ __device__ __forceinline__ int tall_off(int lane, int g, int t) {
 // rows x 64 B ran at half the rate). store(row, tile of the block, gate or
 // plain value, value of the tile after it) takes the results.
 //
-// Folded MXFP4 scales (a.fold) are not used here: with two 32x32x16 MFMAs a
-// product, accumulating inside them would round twice as often as the short
-// tiles' one 16x16x32 does (300 x 8192 x 4096, 64 groups to a running sum:
-// 3.4e-7 from the 64-bit product against 2.0e-7 so).
-//
 // SEG: segq quads at most go into one running sum (see dense_chain,
 // expert.hip). The sums so far are written to this wave's part of a scratch
 // buffer, one set after another (nothing waits for the stores), and added at
 // the end: a second set of accumulators does not fit the registers (spilled
 // inside the loop), and adding to the first set in memory every time waits for
-// it behind the ring's DMAs (the 512-row feed-forward of 4096 x 14336 int4:
-// 397 us as one chain, 480 us with the sums added in memory, SEGTIME so).
+// it behind the ring's DMAs (the 512-row feed-forward of 4096 x 14336 int4: 411
+// us as one chain, 480 us with the sums added in memory, 447 us so).
 //
 // The loop is a sequence of steps, one per (group, row block, column block):
 // the step's 2 (4 with lo parts) MFMAs beside the work that needs no result of
@@ -146,7 +141,7 @@ __device__ __forceinline__ int tall_off(int lane, int g, int t) {
 // on the GEMV kernel, 155 us with the same tiles scheduled by the compiler,
 // 119-139 us here (1.0 PFLOP/s of MFMA work; 1.2 MXFP4; a bf16 library product
 // of 8192^3 reaches 1.4 on the card).
-template <int KIND, bool LO, int NB, bool SEG, typename Store>
+template <int KIND, bool LO, bool FOLD, int NB, bool SEG, typename Store>
 __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, const uint8_t *wt1, const uint8_t *sp,
                                           const _Float16 *xhi, const _Float16 *xlo, uint32_t xo0, uint32_t xo1, int nq,
                                           int segq, float *sums, int lane, int wave, Store store) {
@@ -211,7 +206,8 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
     };
     auto unpack = [&](int n, int t, int j) {
         if (t == 0) scl[j & 1][n] = sc[n].get(j);
-        bw[j & 1][n][t] = unpack_b<KIND>(w[n][t][j]);
+        if constexpr (FOLD) bw[j & 1][n][t] = unpack_fp4_scaled(w[n][t][j], scl[j & 1][n]);
+        else bw[j & 1][n][t] = unpack_b<KIND>(w[n][t][j]);
     };
     const int xofs[2][2] = {{tall_off(lane, 0, 0), tall_off(lane, 0, 1)}, {tall_off(lane, 1, 0), tall_off(lane, 1, 1)}};
     auto load_x = [&](int p, const uint8_t *xs, int g, int b) {   // group g (0, 1) of the half quad, row block b
@@ -225,10 +221,12 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
     auto scale = [&](auto pt, auto bt, auto nt, auto jt) {   // products d[p] of blocks (b, n), group parity jp
         constexpr int p = decltype(pt)::value, b = decltype(bt)::value, n = decltype(nt)::value;
         constexpr int jp = decltype(jt)::value;
-        floatx16 v = acc[b][n];
+        if constexpr (!FOLD) {
+            floatx16 v = acc[b][n];
 #pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = fmaf(d[p][i], scl[jp][n], v[i]);
-        acc[b][n] = v;
+            for (int i = 0; i < 16; i++) v[i] = fmaf(d[p][i], scl[jp][n], v[i]);
+            acc[b][n] = v;
+        }
     };
     auto wait_lds = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
     auto barrier = [&]() {
@@ -288,6 +286,7 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
         // after the ring's synchronization
         if constexpr (half_end ? n == 1 : n == 0) load_x(p ^ 1, aslot(as), (lastb ? j + 1 : j) & 1, lastb ? 0 : b + 1);
         floatx16 z = {};
+        if constexpr (FOLD) z = acc[b][n];
 #pragma unroll
         for (int t = 0; t < 2; t++) z = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[p][t], bw[j & 1][n][t], z, 0, 0, 0);
         if constexpr (LO) {
@@ -295,7 +294,8 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
             for (int t = 0; t < 2; t++)
                 z = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[p][t], bw[j & 1][n][t], z, 0, 0, 0);
         }
-        d[dp] = z;
+        if constexpr (FOLD) acc[b][n] = z;
+        else d[dp] = z;
         // scale the previous step's products (n - 1 of this row block, or n =
         // 1 of the one before)
         constexpr int pb = n == 1 ? b : (b == 0 ? NB - 1 : b - 1), pj = n == 1 || b > 0 ? j : j + 3;
@@ -313,7 +313,7 @@ __device__ __forceinline__ void gemm_tall(uint8_t *lds, const uint8_t *wt0, cons
         }
         // an MFMA first: the wait for this step's operands then comes before
         // the next fragments' reads are queued behind them
-        constexpr int NM = LO ? 4 : 2, NV = (16 + 12 * (4 / NS) + NM - 1) / NM;
+        constexpr int NM = LO ? 4 : 2, NV = FOLD ? 6 / NM : (16 + 12 * (4 / NS) + NM - 1) / NM;
 #pragma unroll
         for (int k = 0; k < NM; k++) {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
@@ -498,17 +498,25 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         if constexpr (SEG)
             sums = a.sums + (size_t)blockIdx.x * ((a.qps - 1) / a.segq) * COLI_GM_SUMS + wave * (COLI_GM_SUMS / COLI_GM_W);
         // the second row half of a tile of up to 96 rows has one row block
-        auto go = [&](auto lo_tag) {
-            constexpr bool LO = decltype(lo_tag)::value;
+        auto go = [&](auto lo_tag, auto fold_tag) {
+            constexpr bool LO = decltype(lo_tag)::value, FOLD = decltype(fold_tag)::value;
             if (nm <= 6 && wave >= 4)
-                gemm_tall<KIND, LO, 1, SEG>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, a.segq, sums, lane,
-                                            wave, put);
+                gemm_tall<KIND, LO, FOLD, 1, SEG>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, a.segq, sums,
+                                                  lane, wave, put);
             else
-                gemm_tall<KIND, LO, 2, SEG>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, a.segq, sums, lane,
-                                            wave, put);
+                gemm_tall<KIND, LO, FOLD, 2, SEG>(lds, wt[0], wt[1], sp, a.xhi, a.xlo, xo[0], xo[1], nq, a.segq, sums,
+                                                  lane, wave, put);
         };
-        if (use_lo) go(std::true_type{});
-        else go(std::false_type{});
+        auto by_fold = [&](auto lo_tag) {
+            if constexpr (KIND == COLI_KIND_FP4 && !SEG) {
+                if (a.fold) go(lo_tag, std::true_type{});
+                else go(lo_tag, std::false_type{});
+            } else {
+                go(lo_tag, std::false_type{});
+            }
+        };
+        if (use_lo) by_fold(std::true_type{});
+        else by_fold(std::false_type{});
         return;
     }
 

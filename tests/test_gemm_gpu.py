@@ -176,8 +176,8 @@ def test_dense_gemm_row_tiles_in_several_launches(session, monkeypatch):
 
 def test_tall_mxfp4_tiles_round_no_more_than_short_ones(session):
     """Eight members of 128 rows (tall tiles) against the same rows as sixteen
-    members of 64 (short tiles, whose folded scales accumulate in the MFMA):
-    the distance from the 64-bit result does not grow. Enough blocks that
+    members of 64 (short tiles); both accumulate folded scales in the MFMA. The
+    distance from the 64-bit result does not grow. Enough blocks that
     gate/up runs without a K split."""
     rng = np.random.default_rng(77)
     D, I = 2048, 4096
