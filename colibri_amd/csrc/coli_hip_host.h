@@ -218,12 +218,12 @@ int run_gemv(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
              const ColiProb *inline_prob = nullptr, float swiglu_limit = 0.0f, const GemvScratch *ws = nullptr,
              GemvEmit *emit = nullptr, bool fold = false);
 // One grouped GEMM over a device work list of (problem << 16 | row tile:
-// COLI_GM_TILE rows, the block-scaled variant's COLI_GM_ROWS), or over one
-// inline problem. split_rows: see expert.hip.
+// `tile` rows, the block-scaled variant's COLI_GM_ROWS), or over one inline
+// problem. split_rows: see expert.hip.
 int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int nprob, const int *nprob_dev,
              const int *mt_list_dev, const int *n_mt_dev, int n_mt, int nrt, int nq, int O, int set,
              const int *xrows_dev, float *out, int ldo, float swiglu_limit = 0.0f, bool fold = false,
-             const ColiProb *inline_prob = nullptr, int split_rows = 0);
+             const ColiProb *inline_prob = nullptr, int split_rows = 0, int tile = COLI_GM_TILE);
 
 // Router logits of S rows into `part`; returns the number of column-chunk
 // partials the selection must add, or 0 on failure.

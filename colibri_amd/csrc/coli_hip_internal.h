@@ -130,7 +130,7 @@ struct ColiGemvArgs {
 #ifndef COLI_GM_ROWS
 #define COLI_GM_ROWS 64     // rows of a short tile (and of the block-scaled variant's tiles)
 #endif
-#define COLI_GM_TILE 128    // rows of a work item of coli_gemm_tiles
+#define COLI_GM_TILE 128    // rows of a tall tile
 #define COLI_GM_SUMS (COLI_GM_TILE * COLI_GM_BLOCK_TILES * 16)   // outputs of a workgroup
 
 struct ColiGemmArgs {
@@ -141,6 +141,7 @@ struct ColiGemmArgs {
     const int *mt_list;       // work list of (problem << 16 | row tile)
     const int *n_mt_dev;      // live entries of mt_list (device)
     int n_mt;                 // upper bound of the list (grid sizing)
+    int tile;                 // rows of a work item: COLI_GM_TILE or COLI_GM_ROWS
     int nrt, nq, O;
     int rb_per_prob;          // output blocks of COLI_GM_WAVES x 2 row tiles (dual: x 1 gate + 1 up)
     const int *xrows;         // fragment row of batch row r = xrows[xrow_off + r] (null: xrow_off + r)

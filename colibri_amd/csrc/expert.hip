@@ -431,7 +431,7 @@ static int dense_chain(const DevCtx *ctx, int nrt, int nq, int S) {
 int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int nprob, const int *nprob_dev,
              const int *mt_list_dev, const int *n_mt_dev, int n_mt, int nrt, int nq, int O, int set,
              const int *xrows_dev, float *out, int ldo, float swiglu_limit, bool fold, const ColiProb *inline_prob,
-             int split_rows) {
+             int split_rows, int tile) {
     if (n_mt <= 0) return 1;
     FragSet &f = ctx->frag[set];
     const bool mx = kind == COLI_KIND_FP4 && !inline_prob && mx_gemm_enabled();
@@ -494,6 +494,7 @@ int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     a.ldo = ldo;
     a.swiglu_limit = swiglu_limit;
     a.fold = fold && kind == COLI_KIND_FP4 && !inline_prob;   // (see dense_chain)
+    a.tile = tile;
     a.splits = 1;
     if (split_rows > 0 && split_rows <= 65535) {
         const long cols = (long)a.rb_per_prob * COLI_GM_BLOCK_TILES * 16;
@@ -629,18 +630,22 @@ static int run_expert_group(DevCtx *ctx, const Member *m, int count, int total, 
     }
     (void)t0g; (void)t0d; (void)split_first;
     // Members of many rows go through the grouped GEMM: one work list of
-    // (problem, row tile) per launch, uploaded after the descriptors.
+    // (problem, row tile) per launch, uploaded after the descriptors, the
+    // members of most rows first: as the last ones their tall tiles would run
+    // on beside an idle chip.
     const bool use_gemm = max_rows > COLI_GEMM_MIN_ROWS;
-    std::vector<int> mt;
+    std::vector<int> mt, order;
     std::vector<int> mt_first(launches.size(), 0), mt_count(launches.size(), 0);
     if (use_gemm)
         for (size_t l = 0; l < launches.size(); l++) {
             mt_first[l] = (int)mt.size();
             const int tile = launches[l].kind == COLI_KIND_FP4 && mx_gemm ? COLI_GM_ROWS : COLI_GM_TILE;
-            for (int q = 0; q < launches[l].n; q++) {
-                const int rows = probs[launches[l].first + q].nrows;
-                for (int t = 0; t * tile < rows; t++) mt.push_back(q << 16 | t);
-            }
+            const ColiProb *lp = &probs[launches[l].first];
+            order.resize(launches[l].n);
+            for (int q = 0; q < launches[l].n; q++) order[q] = q;
+            std::stable_sort(order.begin(), order.end(), [&](int p, int q) { return lp[p].nrows > lp[q].nrows; });
+            for (int q : order)
+                for (int t = 0; t * tile < lp[q].nrows; t++) mt.push_back(q << 16 | t);
             mt_count[l] = (int)mt.size() - mt_first[l];
         }
     if (!probs.empty()) {

@@ -4,7 +4,7 @@
 // the GEMV (c/quant.h fmt=4 and fmt=7) with the weights read once per 128 rows
 // instead of once per 16.
 //
-// Work item = (problem, 128-row tile, output block of COLI_GM_BLOCK_TILES row
+// Work item = (problem, 128-row tile (64: moe_tile_rows, moe.hip), output block of COLI_GM_BLOCK_TILES row
 // tiles, K split). Tiles of more than 64 rows run gemm_tall below (their
 // bound is the matrix cores and the issue slots); shorter ones, whose bound is
 // the weight stream, the loop described here. A K split (only where the host
@@ -416,8 +416,8 @@ __global__ __launch_bounds__(64 * COLI_GM_W) void coli_gemm_tiles(ColiGemmArgs a
         if (p >= a.nprob || (a.nprob_dev && p >= *a.nprob_dev)) return;
     }
     const ColiProb pr = uniform_prob(a.prob ? a.prob[p] : a.prob0);
-    const int m0 = mt * COLI_GM_TILE;
-    const int nrows = min(COLI_GM_TILE, pr.nrows - m0);
+    const int m0 = mt * a.tile;
+    const int nrows = min(a.tile, pr.nrows - m0);
     if (nrows <= 0) return;
     const int Q0 = split * a.qps, nq = min(a.nq, Q0 + a.qps) - Q0;   // this workgroup's quads
 
@@ -822,7 +822,7 @@ extern "C" hipError_t coli_launch_gemm(int kind, int dual, const ColiGemmArgs *a
     if (a->n_mt <= 0 || a->rb_per_prob <= 0) return hipSuccess;
     if ((long)a->n_mt * a->splits * a->rb_per_prob > 0x7fffffffL || (a->prob && !a->mt_list)) return hipErrorInvalidValue;
     // a K split: output rows [0, part_rows) in fragment-row order, at most 65535 of them
-    if (a->splits < 1 || a->qps < 1 || a->segq < 1 || (a->segq < a->qps && (a->prob || (!a->sums && a->prob0.nrows > COLI_GM_ROWS))) || (a->splits > 1 && (!a->partial || a->xrows || a->part_rows < 1 || a->part_rows > 65535)))
+    if ((a->tile != COLI_GM_ROWS && a->tile != COLI_GM_TILE) || a->splits < 1 || a->qps < 1 || a->segq < 1 || (a->segq < a->qps && (a->prob || (!a->sums && a->prob0.nrows > COLI_GM_ROWS))) || (a->splits > 1 && (!a->partial || a->xrows || a->part_rows < 1 || a->part_rows > 65535)))
         return hipErrorInvalidValue;
     switch (kind) {
     case COLI_KIND_I4_H: return launch_gemm_kind<COLI_KIND_I4_H>(*a, dual != 0, st);

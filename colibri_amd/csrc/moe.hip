@@ -359,7 +359,12 @@ __global__ __launch_bounds__(1024) void coli_moe_union(const int *__restrict__ i
     __syncthreads();
     const int nu = s_nu, np = nu + (has_shared ? 1 : 0);
     // packed row and tile offsets in union order: problem tid's exclusive
-    // prefix (np <= 1025: thread 0 takes the shared expert's after the scan)
+    // prefix (np <= 1025: thread 0 takes the shared expert's after the scan).
+    // The shared expert's items (all S rows: tall tiles, about twice a short
+    // one's time) lead the work list; as its last they ran on beside an idle
+    // chip (64 experts, 6 of 512 rows each, int4, 4096 x 1536: 537 -> 507 us). The others stay in union order: an expert's tall and short items
+    // side by side share its weights in the caches (all tall items first: 64
+    // experts of 2048 x 1024 at 2048 rows 649 -> 657 us).
     const int e_of = tid < nu ? order[tid] : -1;
     const int c = e_of >= 0 ? cnt[e_of] : 0, tl = (c + tile - 1) / tile;
     int xc = c, xt = tl;
@@ -383,7 +388,8 @@ __global__ __launch_bounds__(1024) void coli_moe_union(const int *__restrict__ i
         rows += s_ws[v];
         tiles += s_wt[v];
     }
-    const int my_off = pc + xc - c, my_toff = pt + xt - tl;
+    const int sh_tiles = has_shared ? (S + tile - 1) / tile : 0;
+    const int my_off = pc + xc - c, my_toff = sh_tiles + pt + xt - tl;
     if (e_of >= 0) off[e_of] = my_off;
     auto emit = [&](int j, int e, int cn, int o, int to) {
         ColiProb d = tab[2 * e], dn = tab[2 * e + 1];
@@ -399,7 +405,7 @@ __global__ __launch_bounds__(1024) void coli_moe_union(const int *__restrict__ i
         emit(tid, e_of, c, my_off, my_toff);
     }
     if (has_shared) {
-        if (tid == 0) emit(nu, E, S, rows, tiles);
+        if (tid == 0) emit(nu, E, S, rows, 0);
         for (int t = tid; t < S; t += 1024) xrows[rows + t] = t;
     }
     __syncthreads();
@@ -415,7 +421,7 @@ __global__ __launch_bounds__(1024) void coli_moe_union(const int *__restrict__ i
         state[0] = np;
         state[1] = rows + (has_shared ? S : 0);
         state[2] = nu;
-        state[3] = tiles + (has_shared ? (S + tile - 1) / tile : 0);
+        state[3] = tiles + sh_tiles;
     }
 }
 
@@ -1240,6 +1246,19 @@ static int moe_tiles(const ColiHipMoeConfig &c, int S, int tile) {
     return (moe_rows(c, S) + tile - 1) / tile + moe_problems(c, S);
 }
 
+// Rows of a work item of the prefill GEMMs: 128, but 64 where even those, at
+// the average load, are no more than two workgroups a CU in the gate/up launch
+// (one block of 128 outputs each): a tall item takes about twice as long as a
+// short one, and the fewer there are the more CUs wait for it (int4, 2048 x
+// 1024, 16 experts, 2 of 700 rows each: 151 -> 125 us with 64-row items; 8
+// experts, 300 rows: 127 -> 109). With many items the tall form's rate decides:
+// 64 experts, 8 of 2048 rows each, 761 us with 64-row items, 651 with 128.
+static int moe_tile_rows(const DevCtx *ctx, const ColiHipMoeConfig &c, int S) {
+    const long sel = (long)S * c.K, P = std::min((long)c.E, sel), cus = ctx->cu_count ? ctx->cu_count : 256;
+    const long items = std::max(P, sel / COLI_GM_ROWS + P / 2) + (c.has_shared ? (S + COLI_GM_ROWS - 1) / COLI_GM_ROWS : 0);
+    return items * ((c.I + 127) / 128) <= 2 * cus ? COLI_GM_ROWS : COLI_GM_TILE;
+}
+
 // Per-forward buffers for up to S rows (allocated once per growth of S).
 static int moe_reserve(DevCtx *ctx, ColiHipMoe *m, int S) {
     if (S <= m->S_cap) return 1;
@@ -1484,7 +1503,7 @@ static int moe_forward_impl(ColiHipMoe *m, DevCtx *ctx, const float *x_dev, floa
     hipStream_t st = ctx->stream;
     // many-row MXFP4 layers run the block-scaled MFMA GEMM on e4m3 pieces
     const bool gemm = S > COLI_GEMM_MIN_ROWS, mx = gemm && m->kind == COLI_KIND_FP4 && mx_gemm_enabled();
-    const int tile = mx ? COLI_GM_ROWS : COLI_GM_TILE;
+    const int tile = mx ? COLI_GM_ROWS : moe_tile_rows(ctx, c, S);
     // 1. activation fragments, 2-3. router
     if (!(mx ? make_frags8(ctx, fx, x_dev, c.D, S, c.D) : make_frags(ctx, fx, x_dev, c.D, S, c.D, int4))) return 0;
     const int nrt_i = (c.I + 15) / 16, nrt_d = (c.D + 15) / 16;
@@ -1549,7 +1568,7 @@ static int moe_forward_impl(ColiHipMoe *m, DevCtx *ctx, const float *x_dev, floa
     if (gateup_done) {
     } else if (gemm) {
         if (!run_gemm(ctx, m->kind, true, m->pdual, P, m->state, m->mt, m->state + 3, moe_tiles(c, S, tile), nrt_i, nq_d,
-                      c.I, fx, m->xrows, m->h, c.I, c.swiglu_limit, fold))
+                      c.I, fx, m->xrows, m->h, c.I, c.swiglu_limit, fold, nullptr, 0, tile))
             return 0;
     } else if (S == 1 && dual1_enabled() && launch_dual1(m, st, x_dev, nrt_i, nq_d, P, shared_overlap)) {
         if (!hip_check(hipGetLastError(), "moe gate/up")) return 0;
@@ -1600,7 +1619,7 @@ static int moe_forward_impl(ColiHipMoe *m, DevCtx *ctx, const float *x_dev, floa
         return 0;
     if (gemm) {
         if (!run_gemm(ctx, m->kind, false, m->pdown, P, m->state, m->mt, m->state + 3, moe_tiles(c, S, tile), nrt_d, nq_i,
-                      c.D, fh, nullptr, m->y, c.D, 0.0f, fold))
+                      c.D, fh, nullptr, m->y, c.D, 0.0f, fold, nullptr, 0, tile))
             return 0;
     } else if (!run_gemv(ctx, m->kind, false, m->pdown, P, m->state, nrt_d, nq_i, c.D, S, fh, nullptr, m->y, c.D,
                          nullptr, 0.0f, nullptr, nullptr, fold)) {

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from colibri_amd.backend import ColiHipMoeConfig, f32p, i32p, tensor_array
-from moe_ref import Layer, cref, make_router_inputs, moe_reference
+from moe_ref import Layer, cref, free_handles, make_router_inputs, moe_reference
 from quant_util import rand_x, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -214,6 +214,31 @@ def test_moe_layer(session, monkeypatch, fmt, mode, S, shared, plan):
     assert rel_err(out, ref, mag).max() <= TOL
 
 
+@pytest.mark.parametrize("fmt,E,S,shared", [(4, 24, 400, True), (7, 24, 420, False), (4, 6, 330, True),
+                                            (7, 24, 130, True)])
+def test_moe_prefill_item_heights(session, fmt, E, S, shared):
+    """Prefill chunks on either side of the GEMM's item height (two workgroups
+    a CU at 64 rows an item: the first two cases take 128-row items, tall and
+    short ones of an expert, the others 64-row ones), with the shared
+    expert's items at the head of the list."""
+    rng = np.random.default_rng(E + S)
+    D, I, K = 256, 2048, 4
+    layer = Layer(rng, fmt, D, I, E, shared=shared, distinct=4)
+    x, W, b = make_router_inputs(rng, S, D, E, K, 1, bias=True)
+    m, hs = make_moe(session, layer, W, b, K, 1, norm_topk=1)
+    out = np.zeros((S, D), np.float32)
+    idx = np.zeros((S, K), np.int32)
+    try:
+        assert session.b.hip_moe_forward(m, f32p(x), f32p(out), S, i32p(idx), None, None)
+    finally:
+        session.b.hip_moe_free(m)
+        free_handles(session, hs)
+    rows = np.r_[0:8, S // 2, S - 8:S]   # (a sample of the rows; the lists hold all)
+    ri, _, _, ref, mag = moe_reference(layer, x[rows], W, b, K, 1, norm_topk=1)
+    assert np.array_equal(idx[rows], ri), "router top-K indices must be bit-exact"
+    assert rel_err(out[rows], ref, mag).max() <= TOL
+
+
 @pytest.mark.parametrize("case", ["ties", "nan", "few_valid"])
 def test_pipe_router_ties_and_invalid(session, case):
     """Selection order edges (c/backend_cuda.cu:2169-2194, c/route_trace.h:383-393):
@@ -290,8 +315,8 @@ def test_expert_group_without_lo_parts(session, fmt):
                                         (7, False, (114, 140)), (7, True, (114, 140)), (7, False, (100, 150)),
                                         (7, True, (100, 150))])
 def test_expert_group_grouped_gemm(session, fmt, lo, e8):
-    """Members with more than 32 rows run the grouped GEMM (64-row tiles, LDS
-    staged activations): ragged tiles (70 = 64 + 6, 129 = 2 x 64 + 1), a small
+    """Members with more than 32 rows run the grouped GEMM (tiles of up to
+    128 rows, LDS staged activations): ragged tiles (70, 129 = 128 + 1), a small
     member in the same launch, bf16-exact and full f32 activations. MXFP4
     scale exponents inside [114, 140] are folded into the unpacked operand
     (both ends of that range are drawn); a wider range (100 .. 150) keeps the
