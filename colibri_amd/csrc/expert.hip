@@ -383,30 +383,6 @@ int run_gemv(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     return hip_check(coli_launch_gemv(kind, &a, pl.R, dual ? 1 : 0, pl.W, max_rows, ctx->stream), "gemv launch");
 }
 
-// K splits of a grouped GEMM whose work list the host knows, and its time in
-// us: `items` row tiles of at most `tile` rows x rb blocks over nq quads,
-// `rows` output rows of `cols` partial sums each. One workgroup fills a CU, so
-// a launch takes whole rounds of one workgroup per CU; splitting K levels them
-// (and fills a chip that the blocks alone leave idle) for the partials' round
-// trip and the reduction launch. Measured: a workgroup takes about 10 us and
-// 2.5 us a quad on a tall tile, 1.3 us on a short one (224 workgroups of 128 x
-// 256: 11.4 / 20.7 / 95 us at 1 / 4 / 32 quads); the reduction launch about 5
-// us and the partials' bytes, written and read, at about 4 TB/s.
-static double gemm_plan(const DevCtx *ctx, long items, int rb, int nq, int tile, long rows, long cols, int *splits) {
-    const long cus = ctx && ctx->cu_count ? ctx->cu_count : 256;
-    const double tq = tile > COLI_GM_ROWS ? 2.5 : 1.3;
-    double best = 0.0;
-    for (int s = 1; s <= 16 && (s == 1 || nq / s >= 4); s++) {
-        const double us = (double)((items * rb * s + cus - 1) / cus) * (10.0 + (nq + s - 1) / s * tq) +
-                          (s > 1 ? 5.0 + (double)s * rows * cols * 8 / 4e6 : 0.0);
-        if (s == 1 || us < best) {
-            *splits = s;
-            best = us;
-        }
-    }
-    return best;
-}
-
 // Quads of K that the GEMV sums in one running sum for S rows of a dense
 // matrix: its waves (at least four for a single matrix) and K splits each take
 // a share. The GEMM keeps to it for the matrices that dense_on_gemm sends
@@ -421,6 +397,34 @@ static int dense_chain(const DevCtx *ctx, int nrt, int nq, int S) {
     const GemvLaunchPlan g = plan_gemv(ctx, 1, (S + 15) / 16, nrt, nq, false, S);
     const int W = std::max(4, g.W);
     return std::max(1, (g.qps + W - 1) / W);
+}
+
+// K splits of a grouped GEMM whose work list the host knows, and its time in
+// us: `items` row tiles of at most `tile` rows x rb blocks over nq quads,
+// `rows` output rows of `cols` partial sums each. One workgroup fills a CU, so
+// a launch takes whole rounds of one workgroup per CU; splitting K levels them
+// (and fills a chip that the blocks alone leave idle) for the partials' round
+// trip and the reduction launch. Measured: a workgroup takes about 10 us and
+// 2.5 us a quad on a tall tile, 1.3 us on a short one (224 workgroups of 128 x
+// 256: 11.4 / 20.7 / 95 us at 1 / 4 / 32 quads); the reduction launch about 5
+// us and the partials' bytes, written and read, at about 4 TB/s. chain > 0: at
+// most so many quads in one running sum; a tall tile takes 6 us more for each
+// but the last (224 workgroups of 32 quads, three more: 18 us).
+static double gemm_plan(const DevCtx *ctx, long items, int rb, int nq, int tile, long rows, long cols, int chain,
+                        int *splits) {
+    const long cus = ctx && ctx->cu_count ? ctx->cu_count : 256;
+    const double tq = tile > COLI_GM_ROWS ? 2.5 : 1.3;
+    double best = 0.0;
+    for (int s = 1; s <= 16 && (s == 1 || nq / s >= 4); s++) {
+        const int q = (nq + s - 1) / s, sums = chain > 0 && tile > COLI_GM_ROWS ? (q - 1) / chain : 0;
+        const double us = (double)((items * rb * s + cus - 1) / cus) * (10.0 + q * tq + 6.0 * sums) +
+                          (s > 1 ? 5.0 + (double)s * rows * cols * 8 / 4e6 : 0.0);
+        if (s == 1 || us < best) {
+            *splits = s;
+            best = us;
+        }
+    }
+    return best;
 }
 
 // Grouped GEMM over problems of many rows (see gemm.hip); mt_list_dev holds
@@ -496,9 +500,15 @@ int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     a.fold = fold && kind == COLI_KIND_FP4 && !inline_prob;   // (see dense_chain)
     a.tile = tile;
     a.splits = 1;
+    // (int8 activations: every sum is an exact integer, whatever its order)
+    const int chain = inline_prob && !f.nolo ? dense_chain(ctx, nrt, nq, inline_prob->nrows) : 0;
     if (split_rows > 0 && split_rows <= 65535) {
+        // (a group of short members is costed at a tall tile's time too: at
+        // its members' own, it splits K less and measured no faster, 8 x 40
+        // rows of 4096 x 1536 and 16 x 48 of 2048 x 1024 within 3 %)
         const long cols = (long)a.rb_per_prob * COLI_GM_BLOCK_TILES * 16;
-        gemm_plan(ctx, n_mt, a.rb_per_prob, nq, std::min(split_rows, COLI_GM_TILE), split_rows, cols, &a.splits);
+        gemm_plan(ctx, n_mt, a.rb_per_prob, nq, std::min(split_rows, COLI_GM_TILE), split_rows, cols, chain,
+                  &a.splits);
         a.part_rows = split_rows;
         if (a.splits > 1) {
             if (!reserve(ctx, &ctx->partial, (size_t)a.splits * split_rows * cols * sizeof(float), 0)) return 0;
@@ -507,10 +517,8 @@ int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
     }
     a.qps = (nq + a.splits - 1) / a.splits;
     a.splits = (nq + a.qps - 1) / a.qps;
-    // (int8 activations: every sum is an exact integer, whatever its order)
     a.segq = a.qps;
-    if (inline_prob && !f.nolo) {
-        const int chain = dense_chain(ctx, nrt, nq, inline_prob->nrows);
+    if (chain > 0) {
         const int segs = (a.qps + chain - 1) / chain;
         a.segq = (a.qps + segs - 1) / segs;
     }
@@ -986,7 +994,7 @@ static int gemm_rows(DevCtx *ctx, ColiCudaTensor *t, const void *sc, int set, fl
 // rows 42 / 40; 2048 x 7168 128 rows 28 / 37, 192 rows 46 / 40; 512 x 2048
 // 1024 rows 28 / 39. COLI_HIP_GEMV=dma|tiles pins the GEMV here too, =gemm the
 // GEMM (tuning and tests).
-static bool dense_on_gemm(const DevCtx *ctx, const ColiCudaTensor *t, int S) {
+static bool dense_on_gemm(const DevCtx *ctx, const ColiCudaTensor *t, int S, bool exact = false) {
     if (S <= 16) return false;
     if (const char *f = std::getenv("COLI_HIP_GEMV")) {
         if (std::strcmp(f, "gemm") == 0) return true;
@@ -996,7 +1004,8 @@ static bool dense_on_gemm(const DevCtx *ctx, const ColiCudaTensor *t, int S) {
     const int rb = (t->nrt + COLI_GM_BLOCK_TILES - 1) / COLI_GM_BLOCK_TILES;
     int splits;
     const double gemm = gemm_plan(ctx, (S + COLI_GM_TILE - 1) / COLI_GM_TILE, rb, t->nq, std::min(S, COLI_GM_TILE), S,
-                                  (long)rb * COLI_GM_BLOCK_TILES * 16, &splits);
+                                  (long)rb * COLI_GM_BLOCK_TILES * 16, exact ? 0 : dense_chain(ctx, t->nrt, t->nq, S),
+                                  &splits);
     const double gemv = 5.0 + 0.36 * ((S + 15) / 16) * (double)(t->w_bytes + t->sc_bytes) / 1e6;
     return gemm < gemv;
 }
@@ -1119,7 +1128,7 @@ static int idot_dev(DevCtx *ctx, ColiCudaTensor *t, float *y_dev, const float *x
                    "int8 activation rows"))
         return 0;
     const ColiProb p = {t->w, t->sc_unit, nullptr, nullptr, S, 0, 0, 0};
-    if (dense_on_gemm(ctx, t, S) ? !gemm_rows(ctx, t, t->sc_unit, set, (float *)ctx->idot_y.p, S, false)
+    if (dense_on_gemm(ctx, t, S, true) ? !gemm_rows(ctx, t, t->sc_unit, set, (float *)ctx->idot_y.p, S, false)
                                : !run_gemv(ctx, t->kind, false, nullptr, 1, nullptr, t->nrt, t->nq, t->O, S, set,
                                            nullptr, (float *)ctx->idot_y.p, t->O, &p))
         return 0;
