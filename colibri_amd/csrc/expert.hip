@@ -754,7 +754,8 @@ static double now_ms() {
 // it, then one transfer, before: 256 rows of 5120 in and out through an
 // expert, 553 -> 467 us with download_piped; the host's copy takes 70 us and
 // the transfer 102 us each way). Pieces of 512 KiB through copy kernels
-// measured best (DMA-engine copies 1 MiB 501 us, 512 KiB 563).
+// measured best (DMA-engine copies 1 MiB 501 us, 512 KiB 563). src null: the
+// rows are in the buffer already.
 static size_t piece_bytes(size_t bytes) {
     const size_t p = std::max(COLI_PIECE_BYTES, (bytes + COLI_PIECES - 1) / COLI_PIECES);
     return (p + 4095) & ~(size_t)4095;
@@ -764,7 +765,7 @@ static int upload_piped(DevCtx *ctx, void *dst, const PinBuf &pin, const void *s
     const size_t piece = piece_bytes(bytes);
     for (size_t o = 0; o < bytes; o += piece) {
         const size_t n = std::min(piece, bytes - o);
-        std::memcpy((char *)pin.h + o, (const char *)src + o, n);
+        if (src) std::memcpy((char *)pin.h + o, (const char *)src + o, n);
         if (!hip_check(kcopy ? coli_launch_copy_f32((float *)((char *)dst + o), (const float *)((char *)pin.d + o), n / 4,
                                                     ctx->stream)
                              : hipMemcpyAsync((char *)dst + o, (char *)pin.h + o, n, hipMemcpyHostToDevice, ctx->stream),
@@ -777,8 +778,10 @@ static int upload_piped(DevCtx *ctx, void *dst, const PinBuf &pin, const void *s
 // Device rows to the host: the pieces are queued behind the work on the
 // stream and each is copied out of the pinned buffer when it has arrived,
 // while the next one is on its way. Nothing is written to dst before the work
-// that computes the rows has ended without an error.
-static int download_piped(DevCtx *ctx, void *dst, const PinBuf &pin, const void *src, size_t bytes, bool kcopy) {
+// that computes the rows has ended without an error. arrived (or null) is
+// recorded behind the last piece's transfer.
+static int download_piped(DevCtx *ctx, void *dst, const PinBuf &pin, const void *src, size_t bytes, bool kcopy,
+                          hipEvent_t arrived) {
     const size_t piece = piece_bytes(bytes);
     const int n = (int)((bytes + piece - 1) / piece);
     for (; ctx->n_piece_ev < n; ctx->n_piece_ev++)
@@ -795,6 +798,7 @@ static int download_piped(DevCtx *ctx, void *dst, const PinBuf &pin, const void 
             !hip_check(hipEventRecord(ctx->ev_piece[i], ctx->stream), "piece event"))
             return 0;
     }
+    if (arrived) (void)hipEventRecord(arrived, ctx->stream);
     for (int i = 0; i < n; i++) {
         const size_t o = i * piece;
         if (!hip_check(hipEventSynchronize(ctx->ev_piece[i]), "output synchronize")) return 0;
@@ -804,8 +808,10 @@ static int download_piped(DevCtx *ctx, void *dst, const PinBuf &pin, const void 
 }
 
 // Stage host x -> device, run, device y -> pinned host_y (not yet
-// synchronized). Rows of more than a piece each way, with y_host given: out to
-// y_host, synchronized (*done).
+// synchronized). Rows of more than 1 MiB each way, with y_host given: in
+// pieces, and out to y_host, synchronized (*done). With ev (a profiled call)
+// the rows are staged whole before ev[0] and ev[3] lies behind the last
+// transfer, so that the transfer times hold no host copy.
 static int group_stage_and_run(DevCtx *ctx, std::vector<Member> &mem, int count, int total, int D, int I,
                                const float *x, hipEvent_t *ev, float *y_host = nullptr, bool *done = nullptr) {
     size_t xb = (size_t)total * D * sizeof(float);
@@ -815,7 +821,7 @@ static int group_stage_and_run(DevCtx *ctx, std::vector<Member> &mem, int count,
         return 0;
     if (!hip_check(hipStreamSynchronize(ctx->stream), "group staging")) return 0;
     const bool piped = y_host && xb > ((size_t)1 << 20);
-    if (!piped) std::memcpy(ctx->host_x.h, x, xb);
+    if (!piped || ev) std::memcpy(ctx->host_x.h, x, xb);
     if (ev) (void)hipEventRecord(ev[0], ctx->stream);
     // Decode-sized groups cross PCIe in copy kernels that read / write the
     // pinned buffers through their device addresses (measured: the sync group
@@ -824,7 +830,7 @@ static int group_stage_and_run(DevCtx *ctx, std::vector<Member> &mem, int count,
     const char *kc = std::getenv("COLI_HIP_KCOPY");
     const bool kernels = !(kc && kc[0] == '0'), kcopy = kernels && xb <= ((size_t)1 << 20);
     void *hx_dev = ctx->host_x.d, *hy_dev = ctx->host_y.d;
-    if (piped ? !upload_piped(ctx, ctx->x.p, ctx->host_x, x, xb, kernels)
+    if (piped ? !upload_piped(ctx, ctx->x.p, ctx->host_x, ev ? nullptr : x, xb, kernels)
         : kcopy ? !hip_check(coli_launch_copy_f32((float *)ctx->x.p, (const float *)hx_dev, xb / 4, ctx->stream),
                         "group input upload")
               : !hip_check(hipMemcpyAsync(ctx->x.p, ctx->host_x.h, xb, hipMemcpyHostToDevice, ctx->stream),
@@ -836,13 +842,8 @@ static int group_stage_and_run(DevCtx *ctx, std::vector<Member> &mem, int count,
         return 0;
     if (ev) (void)hipEventRecord(ev[2], ctx->stream);
     if (piped) {
-        const int ok = download_piped(ctx, y_host, ctx->host_y, ctx->y.p, xb, kernels);
-        if (ev) {
-            (void)hipEventRecord(ev[3], ctx->stream);
-            (void)hipEventSynchronize(ev[3]);
-        }
-        *done = ok != 0;
-        return ok;
+        *done = download_piped(ctx, y_host, ctx->host_y, ctx->y.p, xb, kernels, ev ? ev[3] : nullptr) != 0;
+        return *done;
     }
     if (kcopy ? !hip_check(coli_launch_copy_f32((float *)hy_dev, (const float *)ctx->y.p, xb / 4, ctx->stream),
                         "group output download")

@@ -21,7 +21,7 @@ import numpy as np
 import pytest
 
 from colibri_amd.backend import f32p, i32p, tensor_array
-from moe_ref import Layer
+from moe_ref import Layer, free_handles
 from oracle_lib import Cref
 from quant_util import deq_i4, deq_mxfp4, magnitude, rand_i4, rand_mxfp4, rand_x, rel_err
 
@@ -248,12 +248,49 @@ def test_upload_fp4_rows16(session, O, I, S):
                                                       ps.ctypes.data_as(C.POINTER(C.c_uint8)), I, O - 1, 0)
 
 
+def test_profiled_transfer_times_hold_no_host_copy(session, monkeypatch):
+    """COLI_CUDA_PROFILE's transfer times of a group call whose rows cross in
+    pieces are the device's alone: host memory that was never touched (a page
+    fault every 4 KiB makes the host's copies several times the transfer)
+    leaves them as they are with touched memory."""
+    import mmap
+    monkeypatch.setenv("COLI_CUDA_PROFILE", "1")
+    b = session.b
+    D, rows = 2048, 7168
+    layer = Layer(np.random.default_rng(5), 4, D, 128, 1)
+    hs = layer.upload(session)
+    arrays = [tensor_array([hs[0][i]]) for i in range(3)]
+    n = (C.c_int * 1)(rows)
+
+    def untouched():
+        m = mmap.mmap(-1, rows * D * 4)
+        m.madvise(mmap.MADV_NOHUGEPAGE)
+        return np.frombuffer(m, np.float32).reshape(rows, D)
+
+    def times(x, y):
+        before, after = ([C.c_double() for _ in range(3)] for _ in range(2))
+        cnt = [C.c_uint64() for _ in range(3)]
+        b.cuda_group_stats(*map(C.byref, cnt), *map(C.byref, before))
+        assert b.cuda_expert_group(*(a[0] for a in arrays), n, 1, f32p(y), f32p(x))
+        b.cuda_group_stats(*map(C.byref, cnt), *map(C.byref, after))
+        return after[0].value - before[0].value, after[2].value - before[2].value
+
+    x, y = np.zeros((rows, D), np.float32) + 0, np.ones((rows, D), np.float32)
+    try:
+        times(x, y)   # (buffers grow on the first call)
+        touched = np.min([times(x, y) for _ in range(3)], axis=0)
+        fresh = np.min([times(untouched(), untouched()) for _ in range(3)], axis=0)
+    finally:
+        free_handles(session, hs)
+    assert (fresh <= 2 * touched).all(), (fresh, touched)
+
+
 @pytest.mark.parametrize("kcopy", ["0", "1"])
 @pytest.mark.parametrize("rows", [[1, 1, 1], [60, 50, 45]])
 def test_expert_group_staging_routes(session, monkeypatch, kcopy, rows):
     """Sync and issue/take group calls bitwise equal under both PCIe staging
     routes (copy kernels on the pinned buffers, DMA copies) and against the
-    oracle; the 155-row group is above the copy-kernel threshold."""
+    oracle; the 155-row group is above 1 MiB each way and crosses in pieces."""
     monkeypatch.setenv("COLI_HIP_KCOPY", kcopy)
     rng = np.random.default_rng(sum(rows) + int(kcopy))
     D, I = 2048, 256
