@@ -45,6 +45,32 @@ def test_grouped_gemm_row_tiles(session, fmt, lo, e8, rows):
         o += r
 
 
+@pytest.mark.parametrize("fmt,lo,e8", [(4, True, None), (4, False, None), (7, True, (114, 140)), (7, False, (100, 150))])
+@pytest.mark.parametrize("rows", [[65, 129], [128, 40], [97, 64, 1]])
+def test_grouped_gemm_split_k(session, fmt, lo, e8, rows):
+    """The same with K split in both launches (17 and 9 quads, few enough
+    blocks to leave the chip idle): tall and short tiles' gate/up partials
+    through the reduction, and output widths (1040, 2064) that end inside a
+    block."""
+    rng = np.random.default_rng(1900 + fmt + 10 * lo + rows[0])
+    D, I = 2064, 1040
+    layer = Layer(rng, fmt, D, I, len(rows), e8_range=e8 or (119, 123))
+    hs = layer.upload(session)
+    x = rng.standard_normal((sum(rows), D)).astype(np.float32) if lo else rand_x(rng, sum(rows), D)
+    try:
+        y = session.expert_group([h[0] for h in hs], [h[1] for h in hs], [h[2] for h in hs], rows, x)
+    finally:
+        for h in hs:
+            for t in h:
+                session.free(t)
+    o = 0
+    for e, r in enumerate(rows):
+        h, ref = layer.expert_forward(e, x[o:o + r])
+        mag = np.abs(h.astype(np.float64)) @ layer.deq(layer.experts[e][2], I)
+        assert rel_err(y[o:o + r], ref, mag).max() <= TOL
+        o += r
+
+
 def upload_dense(session, rng, fmt, half, O, I):
     """(handle, group size, dequantized weights, oracle product)."""
     if fmt == 7:
