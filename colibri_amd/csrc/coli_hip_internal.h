@@ -150,7 +150,6 @@ struct ColiGemmArgs {
     const int *xexp;
     const int *haslo;
     int lo_gen;
-    const uint8_t *zero;
     float *out;
     int ldo;
     float swiglu_limit;       // > 0: DeepSeek-V4 clamped SwiGLU in the DUAL epilogue

@@ -493,7 +493,6 @@ int run_gemm(DevCtx *ctx, int kind, bool dual, const ColiProb *probs_dev, int np
         a.haslo = (const int *)ctx->zeros.p;
         a.lo_gen = 1;
     }
-    a.zero = (const uint8_t *)ctx->zeros.p;
     a.out = out;
     a.ldo = ldo;
     a.swiglu_limit = swiglu_limit;

@@ -60,7 +60,8 @@
 // 16-row subtiles (NM of them, 4 KiB each for the hi half, as much again for
 // lo) and each wave's weight tiles + scales; the ring takes as many stages as
 // the LDS of a CU holds (at most 6), so short tiles stream deeper. One 1 KiB
-// trash slot takes the DMAs of dead chunks (their count per wave stays fixed).
+// trash slot takes the DMAs past a stage's last chunk (their count per wave
+// depends on NM alone).
 template <int KIND>
 struct GmGeom {
     static constexpr int kMt = COLI_GM_ROWS / 16;                 // 16-row subtiles per tile

@@ -1252,7 +1252,8 @@ static int moe_tiles(const ColiHipMoeConfig &c, int S, int tile) {
 // short one, and the fewer there are the more CUs wait for it (int4, 2048 x
 // 1024, 16 experts, 2 of 700 rows each: 151 -> 125 us with 64-row items; 8
 // experts, 300 rows: 127 -> 109). With many items the tall form's rate decides:
-// 64 experts, 8 of 2048 rows each, 761 us with 64-row items, 651 with 128.
+// 64 experts, 8 of 2048 rows each, 761 us before there were tall tiles, 651
+// with them.
 static int moe_tile_rows(const DevCtx *ctx, const ColiHipMoeConfig &c, int S) {
     const long sel = (long)S * c.K, P = std::min((long)c.E, sel), cus = ctx->cu_count ? ctx->cu_count : 256;
     const long items = std::max(P, sel / COLI_GM_ROWS + P / 2) + (c.has_shared ? (S + COLI_GM_ROWS - 1) / COLI_GM_ROWS : 0);
