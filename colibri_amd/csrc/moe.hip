@@ -17,7 +17,7 @@
 // (an expert's rows start at the sum of the earlier experts' counts), so h
 // and y hold S*K (+S) rows whatever the batch. Up to COLI_GEMM_MIN_ROWS rows
 // the experts run the tiled GEMV; beyond, the grouped GEMM over a device-built
-// list of 128-row tiles. Every stage is stream-ordered on the device; nothing
+// list of row tiles. Every stage is stream-ordered on the device; nothing
 // returns to the host between stages, and no stage allocates once the layer
 // has run at a given S.
 #include "coli_hip_host.h"
