@@ -164,3 +164,12 @@ def test_idot_graph_replay_ignores_later_lo_flag(session):
             b.cuda_pipe_free(0, p)
         session.free(h2)
         session.free(h4)
+
+
+@pytest.mark.parametrize("fmt,O,I,S", [(4, 14336, 4096, 200), (7, 8192, 4096, 300), (4, 14336, 4096, 40),
+                                       (4, 4096, 14336, 130)])
+def test_gemm_rows_graph_replays_match_eager(session, monkeypatch, fmt, O, I, S):
+    """The same for dense matrices on the GEMM: the sums put aside in scratch
+    memory by tall tiles, K splits with their reduction, and short tiles."""
+    monkeypatch.setenv("COLI_HIP_GEMV", "gemm")
+    test_gemm_graph_replays_match_eager(session, fmt, O, I, S)
