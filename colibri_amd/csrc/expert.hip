@@ -992,8 +992,9 @@ static int gemm_rows(DevCtx *ctx, ColiCudaTensor *t, const void *sc, int set, fl
 // to 14336 x 4096). Crossovers measured (GEMV / GEMM): 4096 x 14336 17 rows 41
 // / 31 us; 14336 x 4096 32 rows 29 / 27; 4096 x 4096 128 rows 30 / 35, 192
 // rows 42 / 40; 2048 x 7168 128 rows 28 / 37, 192 rows 46 / 40; 512 x 2048
-// 1024 rows 28 / 39. COLI_HIP_GEMV=dma|tiles pins the GEMV here too, =gemm the
-// GEMM (tuning and tests).
+// 1024 rows 28 / 39. exact: int8 activations, whose sums keep to no chain.
+// COLI_HIP_GEMV=dma|tiles pins the GEMV here too, =gemm the GEMM (tuning and
+// tests).
 static bool dense_on_gemm(const DevCtx *ctx, const ColiCudaTensor *t, int S, bool exact = false) {
     if (S <= 16) return false;
     if (const char *f = std::getenv("COLI_HIP_GEMV")) {
